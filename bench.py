@@ -729,10 +729,13 @@ def main():
         etopk = w.extra_indices.shape[-1] if w.extra_indices is not None else 0
         entries = w.extra_k_cache.shape[0] * w.extra_k_cache.shape[1] if w.extra_k_cache is not None else 0
         grid = _native.lib().fgv_sparse_mla_decode_grid(B, SQ, HQ, w.indices.shape[-1], etopk)
-        expanded = query(B, SQ, HQ, w.indices.shape[-1], etopk, entries) > query(B, SQ, HQ, w.indices.shape[-1],
-                                                                                  etopk, 0)
+        need, slots = (query(B, SQ, HQ, w.indices.shape[-1], etopk, n) for n in (entries, 0))
+        # (pieces are not cut when the extra cache is expanded)
+        expanded = entries > 0 and need == entries * 1024 + (0 if grid == 3 else slots)
+        if grid == 3 and expanded:
+            grid = 0
         kernel = {0: "sparse_mla_decode_kernel", 1: "sparse_mla_decode_split_kernel",
-                  2: "sparse_mla_decode_pair_kernel"}[grid]
+                  2: "sparse_mla_decode_pair_kernel", 3: "sparse_mla_decode_pieces_kernel"}[grid]
         workload = (f"mla_{args.mla_case}" + (f"_b{B}" if args.mla_batch else "")
                     + (f"_h{HQ}" if args.mla_heads else ""))
         case = W.MLA_CASES[args.mla_case]

@@ -44,7 +44,9 @@
 // a CU), windows rank their items by list cost, pair long with short, and
 // give the workgroups alone on their CU the longest; up to 4C, windows of 256
 // take their items longest first.  No result bit depends on the order: every
-// item is computed the same way.
+// item is computed the same way.  Few items (a small decode batch) are cut
+// into pieces instead, a workgroup each, whose partial results a second
+// kernel merges.
 //
 // The sparse prefill over bf16 rows (flash_mla_sparse_fwd,
 // sparse_mla_prefill_kernel near the end of the kernels) reuses the attend
@@ -80,6 +82,7 @@ constexpr float kLn2 = 0.693147180559945309f;
 // computed, which bounds the batch.
 constexpr int kSlotFloats = 64 * 512 + 128;
 constexpr int kMaxSplitRows = 8000;
+constexpr int kPieceMinChunks = 2;                            // pieces mode: chunks per piece, at least
 constexpr float kRescaleSlack = 8.0f;                         // log2 of the largest probability
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -121,6 +124,8 @@ struct MlaArgs {
     // C + j share a CU) and the number of windows
     int32_t pair_cus;
     int32_t order_windows;
+    // pieces mode: the most pieces per item, each with a slot of `partials`
+    int32_t pieces;
 };
 
 // K tile addressing: 16-byte block b of row r at r * kKRowBytes + 16 b, rows
@@ -654,12 +659,13 @@ __device__ __forceinline__ void run_segment(const MlaArgs& a, uint8_t (&raw)[2][
     }
 
     if (slot >= 0) {
-        // partial: O as [head][dim] fp32, then the reference maxima and sums
+        // partial: O in the accumulators' own order (each store a whole 1 KiB
+        // of consecutive lanes), then the reference maxima and sums
         float* ws = a.partials + (int64_t)slot * kSlotFloats;
-        float* orow = ws + (wave * 16 + m16) * kHeadDim;
+        float* orow = ws + (wave * 32 * 64 + lane) * 4;
 #pragma unroll
         for (int dt = 0; dt < 32; ++dt)
-            *reinterpret_cast<f32x4_t*>(orow + 16 * dt + 4 * g) = acc[dt];
+            *reinterpret_cast<f32x4_t*>(orow + dt * 64 * 4) = acc[dt];
         if (g == 0) {
             ws[kBlockHeads * kHeadDim + wave * 16 + m16] = m_run;
             ws[kBlockHeads * kHeadDim + kBlockHeads + wave * 16 + m16] = l_run;
@@ -1211,6 +1217,119 @@ sparse_mla_decode_split_kernel(MlaArgs a) {
     }
 }
 
+// ---- Pieces: an item's chunks over several workgroups, for few items.
+//
+// An item is a serial chain of chunks (about 2 us each), so a decode batch of
+// a few rows ran one long chain per row on a few CUs while the others idled.
+// Here an item's chunks are cut into up to a.pieces contiguous runs of at
+// least kPieceMinChunks, one workgroup each; an item of one piece is finished
+// by its workgroup, the others leave fp32 partial slots (item, piece) that
+// sparse_mla_merge_kernel combines in piece order.  The cut depends on the
+// item's own lengths only.  What bounds it now: the first chunk's chain of
+// dependent loads (length, index, cache row) and 128 KiB written and read
+// back per slot.  Measured (graph replays over 3 input sets, us per call):
+// top-k 128 + 512, all lengths full, at 1 / 24 / 100 / 128 rows 62.0 / 72.0 /
+// 74.2 / - -> 31.8 / 54.1 / 66.3 / - with the top-k and index kernels before
+// it, 48.6 -> 42.9 at 128 rows alone; ragged, 24 / 64 / 100 rows 43.5 / 46.6 /
+// 47.5 -> 23.6 / 28.8 / 38.6; 128 + 1856 at 24 rows 134 -> 34.
+__device__ __forceinline__ int item_pieces(const MlaArgs& a, int chunks) {
+    return max(1, min(a.pieces, chunks / kPieceMinChunks));
+}
+
+__global__ void __launch_bounds__(kThreads, 2)
+sparse_mla_decode_pieces_kernel(MlaArgs a) {
+    FGV_MLA_LDS;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int items = gridDim.x / a.pieces;
+    const int piece = blockIdx.x / items, item = blockIdx.x - piece * items;
+    const int bs = item / a.head_blocks, hb = item - bs * a.head_blocks;
+    const int b = bs / a.seq_q, sq = bs - b * a.seq_q;
+    const int n = row_chunks(a, b), s = item_pieces(a, n);
+    if (piece >= s)
+        return;
+    run_segment(a, lds_raw, lds_kbuf, lds_mask, b, sq, hb, n * piece / s, n * (piece + 1) / s,
+                s == 1 ? -1 : item * a.pieces + piece, wave, lane);
+}
+
+// Merges `count` partial slots of one item (slot_of(k) -> its floats, or null
+// for one to skip) by the LSE rule, in order, and writes the item's output.
+// Workgroup `part` (0..15) of the item merges head group part / 4 (16 heads)
+// and dims 128 (part % 4)..+127, wave w two 16-dim tiles of them, in the lane
+// order of the partials: lane (m16, g) holds dims 4g..4g+3 of a tile for head
+// m16.  Four slots are loaded at a time.  A slot that attended nothing has
+// sum 0 and takes weight 0.
+template <typename SlotOf>
+__device__ __forceinline__ void merge_slots(const MlaArgs& a, int b, int sq, int hb, int part, int count,
+                                            SlotOf slot_of) {
+    constexpr int kStat = kBlockHeads * kHeadDim;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, m16 = lane & 15, g = lane >> 4;
+    const int hg = part >> 2, dt = (part & 3) * 8 + 2 * wave;
+    const int hl = hg * 16 + m16, off = ((hg * 32 + dt) * 64 + lane) * 4;
+    float M = -INFINITY;
+    for (int k0 = 0; k0 < count; k0 += 4) {
+        float m[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float* ws = k0 + i < count ? slot_of(k0 + i) : nullptr;
+            m[i] = ws ? ws[kStat + hl] : -INFINITY;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            M = fmaxf(M, m[i]);
+    }
+    const float M_use = M == -INFINITY ? 0.f : M;
+    float L = 0.f;
+    f32x4_t o0 = {0.f, 0.f, 0.f, 0.f}, o1 = o0;
+    for (int k0 = 0; k0 < count; k0 += 4) {
+        float m[4], l[4];
+        f32x4_t r0[4], r1[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float* ws = k0 + i < count ? slot_of(k0 + i) : nullptr;
+            m[i] = l[i] = 0.f;
+            r0[i] = r1[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            if (ws) {
+                m[i] = ws[kStat + hl];
+                l[i] = ws[kStat + kBlockHeads + hl];
+                r0[i] = *reinterpret_cast<const f32x4_t*>(ws + off);
+                r1[i] = *reinterpret_cast<const f32x4_t*>(ws + off + 64 * 4);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float w = l[i] > 0.f ? __builtin_amdgcn_exp2f(m[i] - M_use) : 0.f;
+            L += l[i] * w;
+            o0 += r0[i] * w;
+            o1 += r1[i] * w;
+        }
+    }
+    const int head = hb * kBlockHeads + hl;
+    const bool any = L > 0.f;
+    float factor = 0.f;
+    if (any)
+        factor = a.sink ? 1.f / (L + expf(a.sink[head] - M_use * kLn2)) : 1.f / L;
+    o0 *= factor;
+    o1 *= factor;
+    uint16_t* orow = a.out + b * a.o_sb + sq * a.o_ss + head * a.o_sh + 16 * dt + 4 * g;
+    *reinterpret_cast<uint2*>(orow) = make_uint2(pack_bf16x2(o0[0], o0[1]), pack_bf16x2(o0[2], o0[3]));
+    *reinterpret_cast<uint2*>(orow + 16) = make_uint2(pack_bf16x2(o1[0], o1[1]), pack_bf16x2(o1[2], o1[3]));
+    if (dt == 0 && g == 0)
+        a.lse[b * a.l_sb + head * a.l_sh + sq] = any ? M_use * kLn2 + logf(L) : INFINITY;
+}
+
+// The pieces' merge: 16 workgroups per item.
+__global__ void __launch_bounds__(kThreads)
+sparse_mla_merge_kernel(MlaArgs a) {
+    const int item = blockIdx.x >> 4;
+    const int bs = item / a.head_blocks, hb = item - bs * a.head_blocks;
+    const int b = bs / a.seq_q, sq = bs - b * a.seq_q;
+    const int s = item_pieces(a, row_chunks(a, b));
+    if (s == 1)
+        return;  // finished by its workgroup
+    const float* ws = a.partials + (int64_t)item * a.pieces * kSlotFloats;
+    merge_slots(a, b, sq, hb, blockIdx.x & 15, s, [&](int k) { return ws + (int64_t)k * kSlotFloats; });
+}
+
 // ---- Paired grid: one 8-wave workgroup per CU, both halves on one item.
 //
 // For long lists over more items than CUs but at most two per CU, one 4-wave
@@ -1546,20 +1665,12 @@ sparse_mla_decode_pair_kernel(MlaArgs a) {
 }
 
 // Merges the partial slots of every item that crosses a split range
-// boundary, and writes the items that attend nothing.  Four workgroups per
-// item, one per quarter of its 64 heads; wave w of a workgroup merges 4 head
-// rows, lane l dims 8l..8l+7 of each, so every read of a 2 KiB partial row and
-// every 1 KiB output row is contiguous.  Each slot's reads for the wave's four
-// heads (reference maxima and sums, then the rows) are issued together and
-// unconditionally: a slot whose segment attended nothing holds zero rows and
-// a zero sum, and takes weight 0.
+// boundary, and writes the items that attend nothing: 16 workgroups per item.
 __global__ void __launch_bounds__(kThreads)
 sparse_mla_combine_kernel(MlaArgs a) {
-    constexpr int kHeadsPerWave = kBlockHeads / 4 / (kThreads / 64);
-    const int item = blockIdx.x >> 2, quarter = blockIdx.x & 3;
+    const int item = blockIdx.x >> 4;
     const int R = a.seq_q * a.head_blocks, G = a.split_grid;
     const int b = item / R, jr = item % R;
-    const int sq = jr / a.head_blocks, hb = jr % a.head_blocks;
     const int64_t W = (int64_t)a.row_prefix[a.batch] * R;
     const int n = a.row_prefix[b + 1] - a.row_prefix[b];
     const int64_t p0 = (int64_t)a.row_prefix[b] * R + (int64_t)jr * n, p1 = p0 + n;
@@ -1572,68 +1683,13 @@ sparse_mla_combine_kernel(MlaArgs a) {
         if (k_lo == k_hi)
             return;  // finished by its workgroup
     }
-    auto slot_of = [&](int k) {
-        return a.partials + (int64_t)(k == k_lo ? 2 * k + 1 : 2 * k) * kSlotFloats;
-    };
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int h0 = quarter * (kBlockHeads / 4) + wave * kHeadsPerWave;
-
-    float M[kHeadsPerWave];
-#pragma unroll
-    for (int i = 0; i < kHeadsPerWave; ++i)
-        M[i] = -INFINITY;
-    for (int k = k_lo; k <= k_hi; ++k) {
-        if (start_of(k) == start_of(k + 1))  // skip empty ranges
-            continue;
-        const float* mk = slot_of(k) + kBlockHeads * kHeadDim + h0;
-#pragma unroll
-        for (int i = 0; i < kHeadsPerWave; ++i)
-            M[i] = fmaxf(M[i], mk[i]);
-    }
-    float M_use[kHeadsPerWave], L[kHeadsPerWave];
-    f32x4_t o[kHeadsPerWave][2];
-#pragma unroll
-    for (int i = 0; i < kHeadsPerWave; ++i) {
-        M_use[i] = M[i] == -INFINITY ? 0.f : M[i];
-        L[i] = 0.f;
-        o[i][0] = o[i][1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
-    for (int k = k_lo; k <= k_hi; ++k) {
-        if (start_of(k) == start_of(k + 1))
-            continue;
-        const float* ws = slot_of(k);
-        float m[kHeadsPerWave], l[kHeadsPerWave];
-        f32x4_t r0[kHeadsPerWave], r1[kHeadsPerWave];
-#pragma unroll
-        for (int i = 0; i < kHeadsPerWave; ++i) {
-            m[i] = ws[kBlockHeads * kHeadDim + h0 + i];
-            l[i] = ws[kBlockHeads * kHeadDim + kBlockHeads + h0 + i];
-            const f32x4_t* row = reinterpret_cast<const f32x4_t*>(ws + (h0 + i) * kHeadDim + 8 * lane);
-            r0[i] = row[0];
-            r1[i] = row[1];
-        }
-#pragma unroll
-        for (int i = 0; i < kHeadsPerWave; ++i) {
-            const float w = l[i] > 0.f ? __builtin_amdgcn_exp2f(m[i] - M_use[i]) : 0.f;
-            L[i] += l[i] * w;
-            o[i][0] += r0[i] * w;
-            o[i][1] += r1[i] * w;
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < kHeadsPerWave; ++i) {
-        const int head = hb * kBlockHeads + h0 + i;
-        const bool any = L[i] > 0.f;
-        float factor = 0.f;
-        if (any)
-            factor = a.sink ? 1.f / (L[i] + expf(a.sink[head] - M_use[i] * kLn2)) : 1.f / L[i];
-        const f32x4_t v0 = o[i][0] * factor, v1 = o[i][1] * factor;
-        store16(a.out + b * a.o_sb + sq * a.o_ss + head * a.o_sh + 8 * lane,
-                make_uint4(pack_bf16x2(v0[0], v0[1]), pack_bf16x2(v0[2], v0[3]), pack_bf16x2(v1[0], v1[1]),
-                           pack_bf16x2(v1[2], v1[3])));
-        if (lane == 0)
-            a.lse[b * a.l_sb + head * a.l_sh + sq] = any ? M_use[i] * kLn2 + logf(L[i]) : INFINITY;
-    }
+    merge_slots(a, b, jr / a.head_blocks, jr % a.head_blocks, blockIdx.x & 15, k_hi - k_lo + 1,
+                [&](int i) -> const float* {
+                    const int k = k_lo + i;
+                    if (start_of(k) == start_of(k + 1))  // skip empty ranges
+                        return nullptr;
+                    return a.partials + (int64_t)(k == k_lo ? 2 * k + 1 : 2 * k) * kSlotFloats;
+                });
 }
 
 // Dequantises every entry of a list's cache into bf16 rows [num_entries][512]
@@ -1739,7 +1795,7 @@ int64_t chunks_of(int64_t topk) { return (topk + kChunk - 1) / kChunk; }
 int split_grid() { return 2 * cu_count(); }
 
 // The grids (fgv_sparse_mla_decode_grid's values).
-enum MlaGrid { kGridOneItem = 0, kGridSplit = 1, kGridPair = 2 };
+enum MlaGrid { kGridOneItem = 0, kGridSplit = 1, kGridPair = 2, kGridPieces = 3 };
 
 int64_t items_of(int64_t batch, int64_t seq_q, int64_t num_heads) { return batch * seq_q * (num_heads / kBlockHeads); }
 
@@ -1761,12 +1817,40 @@ bool pair_fits(int64_t batch, int64_t items, int64_t topk, int64_t extra_topk) {
     return long_lists(batch, items, topk, extra_topk) && items > cus && items <= 2 * cus && items <= kPairMaxItems;
 }
 
-// The grid a call runs when it gets the workspace it asks for.
+// Pieces per item (1: no cut).  Lists shorter than the split grid's but of
+// more than kPieceMinTotal chunks, over at most half as many items as CUs (at
+// most as many, for lists of kPieceLongChunks), are cut so that about one
+// workgroup per CU (two, for the latter) has work, if the chunks that leave
+// the chain are worth the slots: a chunk off the chain saves about 2.1 us, the
+// merge costs about 4 us and 0.06 us per slot (measured from 2 to 496 slots).
+// 128 + 192 entries at 2 / 24 / 100 rows: 25.3 -> 13.8, 26.2 -> 23.6, and 27.6
+// against 30.7 us cut, which the rule leaves whole; 128 + 512 at 130 / 200
+// rows 48.7 / 49.3 against 45.9 / 55.3 us in two pieces, left whole; 128 +
+// 1024 at 100 / 200 rows 81.4 / 82.6 us whole, 57.5 / 82.7 with one workgroup
+// per CU and 51.3 / 76.1 with two, while 24 rows take 30.2 with one and 34.7
+// with two.
+constexpr int64_t kPieceMinTotal = 8;
+constexpr int64_t kPieceLongChunks = 32;
+constexpr int64_t kPieceMaxSlots = 496;  // with their headers below the no-allocation entry point's 64 MiB
+
+int64_t pieces_of(int64_t items, int64_t topk, int64_t extra_topk) {
+    const int64_t chunks = chunks_of(topk) + chunks_of(extra_topk), cus = cu_count();
+    if (chunks <= kPieceMinTotal || chunks >= kSplitMinChunks || items > cus)
+        return 1;
+    const bool two = 4 * items > cus && chunks >= kPieceLongChunks;
+    const int64_t n = min(min(two ? 2 * cus : cus, kPieceMaxSlots) / items, chunks / kPieceMinChunks);
+    return n > 1 && 35 * chunks * (n - 1) > n * (67 + n * items) ? n : 1;
+}
+
+// The grid a call runs when it gets the workspace it asks for (a call whose
+// extra cache is expanded keeps one workgroup per item).
 int mla_grid(int64_t batch, int64_t seq_q, int64_t num_heads, int64_t topk, int64_t extra_topk) {
     const int64_t items = items_of(batch, seq_q, num_heads);
     if (pair_fits(batch, items, topk, extra_topk))
         return kGridPair;
-    return long_lists(batch, items, topk, extra_topk) ? kGridSplit : kGridOneItem;
+    if (long_lists(batch, items, topk, extra_topk))
+        return kGridSplit;
+    return pieces_of(items, topk, extra_topk) > 1 ? kGridPieces : kGridOneItem;
 }
 
 // An extra list gathered at least this many times per cache entry (counting
@@ -1785,8 +1869,15 @@ int64_t expand_bytes(int64_t batch, int64_t seq_q, int64_t num_heads, int64_t ex
     return gathers >= kExpandMinReuse * extra_entries ? extra_entries * 2 * kHeadDim : 0;
 }
 
-int64_t split_bytes(int64_t batch, int64_t seq_q, int64_t num_heads, int64_t topk, int64_t extra_topk) {
-    if (mla_grid(batch, seq_q, num_heads, topk, extra_topk) != kGridSplit)
+// The partial slots of the split grid or of the pieces, with the split's row
+// prefix sums.  `expanded`: the call's extra cache is expanded.
+int64_t split_bytes(int64_t batch, int64_t seq_q, int64_t num_heads, int64_t topk, int64_t extra_topk, bool expanded) {
+    const int grid = mla_grid(batch, seq_q, num_heads, topk, extra_topk);
+    if (grid == kGridPieces && !expanded) {
+        const int64_t items = items_of(batch, seq_q, num_heads);
+        return items * pieces_of(items, topk, extra_topk) * kSlotFloats * 4;
+    }
+    if (grid != kGridSplit)
         return 0;
     const int64_t slots = 2 * (int64_t)split_grid() * kSlotFloats * 4;
     return slots + ((batch + 1) * 4 + 255) / 256 * 256;
@@ -1801,8 +1892,8 @@ extern "C" int64_t fgv_sparse_mla_decode_workspace_bytes(int64_t batch, int64_t 
     if (batch <= 0 || seq_q <= 0 || num_heads <= 0 || num_heads % fgv::kBlockHeads || topk < 0 || extra_topk < 0 ||
         extra_num_entries < 0)
         return 0;
-    return fgv::expand_bytes(batch, seq_q, num_heads, extra_topk, extra_num_entries) +
-           fgv::split_bytes(batch, seq_q, num_heads, topk, extra_topk);
+    const int64_t expand = fgv::expand_bytes(batch, seq_q, num_heads, extra_topk, extra_num_entries);
+    return expand + fgv::split_bytes(batch, seq_q, num_heads, topk, extra_topk, expand > 0);
 }
 
 extern "C" int fgv_sparse_mla_decode_grid(int64_t batch, int64_t seq_q, int64_t num_heads, int64_t topk,
@@ -1891,14 +1982,16 @@ int mla_decode(FGV_MLA_PARAMS, void* workspace, int64_t workspace_bytes, void* s
     a.split_grid = 0;
     a.pair_cus = 0;
     a.order_windows = 0;
+    a.pieces = 0;
     const int64_t items = batch * seq_q * a.head_blocks;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    // Workspace: [expanded extra cache][split slots][row prefix sums].  A
+    // Workspace: [expanded extra cache][partial slots][row prefix sums].  A
     // workspace too small for both drops the expansion first, then the split.
-    // (the combine kernel runs four workgroups per item)
-    const int64_t need_split = split_bytes(batch, seq_q, num_heads, topk, extra_k_cache ? extra_topk : 0);
+    // (the combine and merge kernels run 16 workgroups per item)
     const int64_t need_expand =
         extra_k_cache ? expand_bytes(batch, seq_q, num_heads, extra_topk, a.list[1].num_entries) : 0;
+    const int64_t need_split =
+        split_bytes(batch, seq_q, num_heads, topk, extra_k_cache ? extra_topk : 0, need_expand > 0);
     const int64_t have = workspace ? workspace_bytes : 0;
     const bool use_expand = need_expand > 0 && have >= need_expand + need_split;
     const bool use_split = need_split > 0 && have >= need_split + (use_expand ? need_expand : 0);
@@ -1920,6 +2013,17 @@ int mla_decode(FGV_MLA_PARAMS, void* workspace, int64_t workspace_bytes, void* s
             return rc;
         ws += need_expand;
     }
+    if (use_split && mla_grid(batch, seq_q, num_heads, topk, extra_k_cache ? extra_topk : 0) == kGridPieces) {
+        a.pieces = (int32_t)pieces_of(items, topk, extra_k_cache ? extra_topk : 0);
+        a.partials = reinterpret_cast<float*>(ws);
+        hipLaunchKernelGGL(sparse_mla_decode_pieces_kernel, dim3((unsigned)(items * a.pieces)), dim3(kThreads), 0, st,
+                           a);
+        rc = launch_status();
+        if (rc)
+            return rc;
+        hipLaunchKernelGGL(sparse_mla_merge_kernel, dim3((unsigned)(16 * items)), dim3(kThreads), 0, st, a);
+        return launch_status();
+    }
     if (use_split) {
         a.split_grid = split_grid();
         a.partials = reinterpret_cast<float*>(ws);
@@ -1928,7 +2032,7 @@ int mla_decode(FGV_MLA_PARAMS, void* workspace, int64_t workspace_bytes, void* s
         rc = launch_status();
         if (rc)
             return rc;
-        hipLaunchKernelGGL(sparse_mla_combine_kernel, dim3((unsigned)(4 * items)), dim3(kThreads), 0, st, a);
+        hipLaunchKernelGGL(sparse_mla_combine_kernel, dim3((unsigned)(16 * items)), dim3(kThreads), 0, st, a);
         return launch_status();
     }
     if (pair_fits(batch, items, topk, extra_k_cache ? extra_topk : 0)) {

@@ -376,7 +376,7 @@ int fgv_sparse_mla_decode_model1(
 
 /*
  * Bytes of device workspace (256-byte aligned) that fgv_sparse_mla_decode_model1
- * can use, the sum of two optional parts:
+ * can use, the sum of optional parts:
  *   - an expanded extra cache: when the extra list is gathered at least 8 times
  *     per cache entry (batch * seq_q * num_heads/64 * extra_topk >=
  *     8 * extra_num_entries) and the copy is at most 64 MiB, the extra cache is
@@ -388,7 +388,12 @@ int fgv_sparse_mla_decode_model1(
  *     CU splits all items' chunks evenly, and a combine kernel merges the
  *     items that cross a split (the reference's split-KV schedule and
  *     combine, ops/flash_mla_with_kvcache_model1.py:1212-1395).  Its size
- *     depends on the current device's CU count.
+ *     depends on the current device's CU count;
+ *   - or the partial slots of pieces: lists of 9 to 63 32-entry chunks over few
+ *     items (at most one per CU, or half as many) whose extra cache is not
+ *     expanded are cut into up to one or two pieces per CU, and a merge kernel
+ *     combines them.  At most 496 slots, which also fit the 64 MiB scratch of
+ *     the no-allocation entry point.
  * extra_num_entries is extra_num_blocks * extra_page_size (0 without an extra
  * cache).  0 means the workspace argument is ignored.  Passing no workspace
  * (NULL or too small) always works: a workspace too small for both parts drops
@@ -407,7 +412,10 @@ int64_t fgv_sparse_mla_decode_workspace_bytes(int64_t batch, int64_t seq_q, int6
  *   2  the paired grid (sparse_mla_decode_pair_kernel): lists as long as the
  *      split grid's over more items than CUs but at most two per CU (and at
  *      most 512); one 8-wave workgroup per CU attends each of its items with
- *      both halves, a short item after a long one, and writes no partials.
+ *      both halves, a short item after a long one, and writes no partials;
+ *   3  items cut into pieces and their merge (sparse_mla_decode_pieces_kernel,
+ *      sparse_mla_merge_kernel): lists of 9 to 63 chunks over few items; a
+ *      call whose extra cache is expanded takes 0 instead.
  * -1 for sizes the decode rejects.  No counterpart in the reference: it is
  * for benchmarks, profilers and tests that need the kernel's name.
  */

@@ -1017,3 +1017,63 @@ def _longest_first_case(name):
 def test_gpu_longest_first_order_against_oracle(case):
     print(f"\n[case] sparse MLA one-item grid, longest first, {case}", flush=True)
     _check_item_order(_longest_first_case(case), case, case != "extra_fp8", (2, 4))
+
+
+# --------------------------------------------- GPU: pieces of few items ----
+
+def _pieces_case(name):
+    """Calls that cut their items into pieces: 9 to 63 chunks over few items."""
+    if name == "least":       # 9 chunks, one row
+        return W.make_mla_workload(batch=1, topk=256, num_pages=16, extra_topk=64, extra_page=64, extra_pages=40,
+                                   topk_length=False, seed=91, q_scale=0.1)
+    if name == "most":        # 63 chunks, 128 heads, two query positions
+        return W.make_mla_workload(batch=2, topk=64, num_pages=16, heads=128, seq_q=2, extra_topk=1920,
+                                   extra_page=2, extra_pages=4000, seed=92, q_scale=0.1)
+    # a ragged batch at the most items of its rule; rows of every remainder, empty ones and single chunks
+    batch, extra = {"half": (128, 512), "all": (224, 1024), "few": (24, 512)}[name]
+    w = W.make_mla_workload(batch=batch, topk=128, num_pages=32, extra_topk=extra, extra_page=64, extra_pages=500,
+                            seed=93 + batch, q_scale=0.1)
+    w.topk_length = _lengths(batch, 128, 11)
+    w.extra_topk_length = _lengths(batch, extra, 12)
+    w.topk_length[:6] = torch.tensor([0, 0, 1, 33, 128, 128], dtype=torch.int32)
+    w.extra_topk_length[:6] = torch.tensor([0, 1, 0, 0, extra, extra - 31], dtype=torch.int32)
+    return w
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ["least", "most", "half", "all", "few"])
+def test_gpu_pieces_against_oracle(case):
+    """Items cut into pieces and merged: within the bound of the binary64
+    oracle, and the LSE at binary32 precision, as the uncut call (without a
+    workspace) is."""
+    print(f"\n[case] sparse MLA pieces {case}", flush=True)
+    w = _pieces_case(case)
+    assert _grid(w) == 3
+    out, lse, nbytes = _gpu_raw(w, workspace=True)
+    items = w.q.shape[0] * w.q.shape[1] * (w.q.shape[2] // 64)
+    assert nbytes % (items * (64 * 512 + 128) * 4) == 0 and 0 < nbytes < 64 << 20
+    o64, l64 = _oracle(w)
+    fin = torch.isfinite(l64)
+    for o, l, what in ((out, lse, case), (*_gpu_raw(w, workspace=False)[:2], case + " uncut")):
+        _assert_within_bound(o, o64, _vmax(w), what)
+        assert torch.equal(torch.isfinite(l), fin), what
+        assert torch.allclose(l.double()[fin], l64[fin], rtol=1e-5, atol=1e-5), what
+
+
+def test_pieces_rule():
+    """Where items are cut, and that what the query asks for is bounded."""
+    from flaggems_vllm import _native
+
+    f = _native.lib().fgv_sparse_mla_decode_workspace_bytes
+    grid = _native.lib().fgv_sparse_mla_decode_grid
+    slot = (64 * 512 + 128) * 4
+    assert grid(24, 1, 64, 128, 512) == 3 and f(24, 1, 64, 128, 512, 1 << 20) == 24 * 10 * slot
+    assert grid(24, 1, 64, 256, 0) == 0 and f(24, 1, 64, 256, 0, 0) == 0          # 8 chunks: whole
+    assert grid(128, 1, 64, 128, 512) == 3 and grid(129, 1, 64, 128, 512) == 0    # more items than half the CUs
+    assert grid(248, 1, 64, 128, 1024) == 3 and grid(256, 1, 64, 128, 1024) == 0  # long: two pieces each fit
+    assert grid(100, 1, 64, 128, 192) == 0                                        # not worth the slots
+    assert f(24, 1, 64, 128, 512, 1000) == 1000 * 1024                            # expanded: not cut
+    for batch in range(1, 257):
+        for extra in (0, 192, 512, 1024, 1888):
+            for heads in (64, 128):
+                assert f(batch, 1, heads, 128, extra, 1 << 20) <= 64 << 20 or grid(batch, 1, heads, 128, extra) == 1
