@@ -271,21 +271,9 @@ __global__ void __launch_bounds__(64 * KS) fp8_einsum_skinny_kernel(EinsumArgs a
 constexpr int kStages4 = 3;  // LDS stages of the 256-row tiles (49 KB each)
 constexpr int kStages2 = 3;  // LDS stages of the 128-row tiles (33 KB each)
 
-// LDS DMA of 16 (4) bytes per lane: lane l's bytes land at LDS address
-// lds + 16 l (4 l).  Issued as inline assembly so that the compiler, which
-// cannot tell the stages apart, does not wait for every DMA in flight before
-// each LDS read; the kernel waits for its own (vmcnt) and has no other vector
-// memory loads in flight while DMAs are.
-__device__ __forceinline__ void dma16(const void* src, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds) : "memory", "m0");
-}
-__device__ __forceinline__ void dma4(const void* src, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(lds) : "memory", "m0");
-}
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-
+// The kernel's LDS DMAs are fgv_device.h's dma16 / dma4: the compiler does not
+// know of them, so the kernel waits for its own (vmcnt) and has no other vector
+// memory loads in flight while they are.
 __device__ __forceinline__ int swz(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
 
 // s_waitcnt operand: vector memory operations outstanding <= n (expcnt and

@@ -13,7 +13,7 @@
 // the extra list, stream through in chunks of 32 with a three-stage pipeline:
 //   - the index each lane needs for chunk c+2 is loaded into a register,
 //   - the raw 576 token bytes and 8 scale bytes of each entry of chunk c+1 are
-//     gathered straight into LDS (global_load_lds_dwordx4: no registers, no
+//     gathered straight into LDS (dma16: no registers, no
 //     wait), into the other half of a double buffer; 8 lanes move one entry,
 //     so each lane resolves one index per chunk,
 //   - chunk c, gathered one iteration earlier, is dequantised from LDS into a
@@ -89,8 +89,6 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) short4_t lds_short4_t;
-typedef __attribute__((address_space(3))) uint32_t lds_u32_t;
-typedef const __attribute__((address_space(1))) uint32_t global_u32_t;
 
 struct CacheList {
     const uint8_t* cache;
@@ -263,20 +261,19 @@ __device__ __forceinline__ int64_t entry_offset(const ListView& v, int id, int64
 // after the wait at the top of the next chunk.
 __device__ __forceinline__ void issue_gather(const ListView& v, const uint8_t* dummy, int wave, int lane, int id,
                                              uint8_t* raw, float* mask) {
-    __attribute__((address_space(3))) uint8_t* dst = (__attribute__((address_space(3))) uint8_t*)raw;
+    const uint32_t dst = lds_addr(raw);
     const int e = 8 * wave + (lane >> 3), sub = lane & 7;
     const int64_t off = entry_offset(v, id, kTokenDataBytes);
     const uint8_t* tok = off >= 0 ? v.cache + off : dummy;
 #pragma unroll
     for (int n = 0; n < kGathers; ++n) {
         const int k = sub + 8 * n < kPieces ? sub + 8 * n : kPieces - 1;
-        __builtin_amdgcn_global_load_lds((global_u32_t*)(tok + 16 * k),
-                                         (lds_u32_t*)(dst + n * kRegion + 1024 * wave), 16, 0, 0);
+        dma16(tok + 16 * k, dst + n * kRegion + 1024 * wave);
     }
     const int64_t soff = entry_offset(v, id, kScaleBytesPerToken);
     const uint8_t* scl = (soff >= 0 ? v.cache + (int64_t)v.page_size * kTokenDataBytes + soff : mla_unit_scales) +
                          4 * (lane & 1);
-    __builtin_amdgcn_global_load_lds((global_u32_t*)scl, (lds_u32_t*)(dst + kRawScaleOff + 256 * wave), 4, 0, 0);
+    dma4(scl, dst + kRawScaleOff + 256 * wave);
     if (sub == 0)
         mask[e] = off >= 0 ? 0.f : -INFINITY;
 }
@@ -289,7 +286,7 @@ __device__ __forceinline__ void issue_gather(const ListView& v, const uint8_t* d
 // mask is written as for a gather.
 __device__ __forceinline__ void issue_rows(const ListView& v, int wave, int lane, int id, uint8_t* tile,
                                            float* mask) {
-    __attribute__((address_space(3))) uint8_t* dst = (__attribute__((address_space(3))) uint8_t*)tile;
+    const uint32_t dst = lds_addr(tile);
     const int src_off = 16 * lane;
     // each lane forms its entry's row address once; row j's is read from lane 8j
     const uint8_t* mine = id >= 0 && id < v.num_entries ? v.expanded + (int64_t)id * (2 * kHeadDim) : mla_zero_entry;
@@ -299,8 +296,7 @@ __device__ __forceinline__ void issue_rows(const ListView& v, int wave, int lane
         const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)maddr, 8 * j);
         const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(maddr >> 32), 8 * j);
         const uint8_t* row = reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
-        __builtin_amdgcn_global_load_lds((global_u32_t*)(row + src_off),
-                                         (lds_u32_t*)(dst + (8 * wave + j) * kKRowBytes), 16, 0, 0);
+        dma16_row(row, src_off, dst + (8 * wave + j) * kKRowBytes);
     }
     if ((lane & 7) == 0)
         mask[8 * wave + (lane >> 3)] = id >= 0 && id < v.num_entries ? 0.f : -INFINITY;
@@ -353,10 +349,8 @@ __device__ __forceinline__ void dequantize(const uint8_t* raw, uint8_t* kbuf, in
 }
 
 // The workgroup's LDS: the double-buffered raw gather, the bf16 K tile, the
-// gathered indices and the score masks.  They are separate __shared__ arrays
-// (declared in each kernel, passed down by reference) so that the compiler
-// can tell the LDS-DMA targets from the tile the MFMAs read; as members of
-// one object they would make every tile read wait for the gathers.
+// gathered indices and the score masks, as separate __shared__ arrays
+// (declared in each kernel, passed down by reference).
 #define FGV_MLA_LDS                                              \
     __shared__ __align__(16) uint8_t lds_raw[2][kRawBytes];      \
     __shared__ __align__(16) uint8_t lds_kbuf[kChunk * kKRowBytes]; \
@@ -399,8 +393,6 @@ __device__ __forceinline__ void lds_barrier() {
 // fp32 O^T accumulators, m_run / l_run the reference maximum (base 2) and the
 // running sum.  qk_base / tr_base are the lane's K-tile byte offsets for the
 // QK row reads and the PV transposing reads, g its 16-lane group.
-// (Each call site passes one fixed LDS array, so the compiler can tell the
-// tile read from the tile the LDS DMA is filling.)
 //
 // With TAIL, the scores have 64 more dims (the sparse prefill's d_qk = 576):
 // q's in qt (lane group g: dims 512+32t+8g..+7 of step t), the entries' in
@@ -988,7 +980,7 @@ struct PrefillArgs {
 template <bool TAIL>
 __device__ __forceinline__ void issue_kv_rows(const PrefillArgs& a, int wave, int lane, int id, uint8_t* tile,
                                               uint8_t* tail, float* mask) {
-    __attribute__((address_space(3))) uint8_t* dst = (__attribute__((address_space(3))) uint8_t*)tile;
+    const uint32_t dst = lds_addr(tile);
     // every lane forms its entry's row address once (vector ALU); row j's
     // address is then read from lane 8j, with no scalar arithmetic or branch
     // per row
@@ -1000,14 +992,11 @@ __device__ __forceinline__ void issue_kv_rows(const PrefillArgs& a, int wave, in
         const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)maddr, 8 * j);
         const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(maddr >> 32), 8 * j);
         const uint8_t* row = reinterpret_cast<const uint8_t*>(((uint64_t)hi << 32) | lo);
-        __builtin_amdgcn_global_load_lds((global_u32_t*)(row + 16 * lane),
-                                         (lds_u32_t*)(dst + (8 * wave + j) * kKRowBytes), 16, 0, 0);
+        dma16_row(row, 16 * lane, dst + (8 * wave + j) * kKRowBytes);
     }
     if constexpr (TAIL) {
-        __attribute__((address_space(3))) uint8_t* tdst = (__attribute__((address_space(3))) uint8_t*)tail;
         const uint8_t* row = valid ? mine + 2 * kHeadDim : mla_zero_entry;
-        __builtin_amdgcn_global_load_lds((global_u32_t*)(row + 16 * (lane & 7)),
-                                         (lds_u32_t*)(tdst + 8 * kTailRow * wave), 16, 0, 0);
+        dma16(row + 16 * (lane & 7), lds_addr(tail) + 8 * kTailRow * wave);
     }
     if ((lane & 7) == 0)
         mask[8 * wave + (lane >> 3)] = valid ? 0.f : -INFINITY;
@@ -1426,8 +1415,7 @@ sparse_mla_decode_pair_kernel(MlaArgs a) {
 #pragma unroll
         for (int L = 0; L < 2; ++L)
             if (L < a.num_lists && a.list[L].lengths)
-                __builtin_amdgcn_global_load_lds((global_u32_t*)(a.list[L].lengths + i / R),
-                                                 (lds_u32_t*)&lds_len[L][64 * wave], 4, 0, 0);
+                dma4(a.list[L].lengths + i / R, lds_addr(&lds_len[L][64 * wave]));
     }
     auto item_chunks = [&](int i) {
         const int t0 = a.list[0].topk, t1 = a.list[1].topk;
