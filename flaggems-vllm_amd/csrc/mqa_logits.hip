@@ -306,22 +306,23 @@ struct PagedArgs {
     int64_t o_sr;          // float elements
     int32_t rows, bt_row_div, ctx_row_div;
     int32_t num_blocks, block_size, max_blocks;
-    int32_t max_model_len, keys_per_block;  // keys_per_block: multiple of 1024
+    int32_t max_model_len;
+    int32_t block_shift;                    // log2 of block_size where that is a power of two (SHIFT)
     int32_t vec_fill;                       // output rows 16-byte aligned, max_model_len % 4 == 0
     float fill;
 };
 
-// Paged logits: one workgroup per (row, keys_per_block positions); each wave
-// takes 64 consecutive positions at a time: all four key tiles' cache loads
-// are issued before the first tile is multiplied.
-template <bool FP4, int HT>
+// Paged logits: one workgroup per (row, kPagedKeys positions).
+constexpr int kPagedKeys = 1024;
+template <bool FP4, int HT, bool SHIFT>
 __global__ void __launch_bounds__(kThreadsM, 2)
 paged_mqa_logits_kernel(PagedArgs a) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int c = lane & 15, g = lane >> 4;
+    constexpr int kSteps = kPagedKeys / kThreadsM;
     const int row = blockIdx.y;
-    const int n_begin = blockIdx.x * a.keys_per_block;
-    const int n_end = min(a.max_model_len, n_begin + a.keys_per_block);
+    const int n_begin = blockIdx.x * kPagedKeys;
+    const int n_end = min(a.max_model_len, n_begin + kPagedKeys);
     const int ctx = min(max(a.ctx[row / a.ctx_row_div], 0), a.max_model_len);
     float* out = a.out + (int64_t)row * a.o_sr;
     if (n_begin >= ctx) {
@@ -340,40 +341,74 @@ paged_mqa_logits_kernel(PagedArgs a) {
             a.w + (int64_t)row * a.w_sr, a.w_sh, c, g);
     const int32_t* bt_row = a.bt + (int64_t)(row / a.bt_row_div) * a.bt_sr;
     const int64_t scale_off = (int64_t)a.block_size * kIdxDim;
-    // each wave: positions n0 .. n0 + 63 per step, the four key tiles' cache
-    // loads issued before the first MFMA.  (A two-stage pipeline, the next
-    // step's loads issued before the current one is multiplied, measured 1.6x
-    // slower: 184 VGPRs halve the waves per SIMD.)
-    for (int n0 = n_begin + 64 * wave; n0 < n_end; n0 += 256) {
-        v8i_t b[4];
-        float ksc[4];
+    // A wave takes 64 positions (four 16-key tiles) per step, kSteps steps.  The
+    // block-table entries of every step are loaded first, together; each key
+    // tile's registers then take the next step's tile as soon as the tile's own
+    // MFMAs have read them, so three tiles' loads are in flight under each
+    // tile's MFMAs and gate, with the registers of one step.  Positions from ctx
+    // on read position ctx - 1 (they are not stored).  What bounds it: the
+    // keys' HBM stream.  32 rows x 65536 positions 77.7 -> 71.8 us, 256 x 8192
+    // 81.3 -> 78.3, 4 x 2 x 3000 10.3 -> 7.8 (against all four tiles' table entries and keys loaded, then
+    // multiplied; a second step's tiles in registers of their own measured
+    // 1.6x slower than that: 184 VGPRs; the 174 here held to 168 spill: 121 us).
+    const int w0 = n_begin + 64 * wave, last = ctx - 1;
+    auto block_of = [&](int n) { return SHIFT ? n >> a.block_shift : (int)((uint32_t)n / (uint32_t)a.block_size); };
+    int blk[2][4];  // of this step and the next
+    auto look_up = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
-            const int n = n0 + 16 * kt + c;
-            if (n < ctx) {
-                const int lbn = (int)((uint32_t)n / (uint32_t)a.block_size);
-                const int slot = n - lbn * a.block_size;
-                // positions past the table read its last block (the table index is clamped)
-                const int blk = min(max(bt_row[min(lbn, a.max_blocks - 1)], 0), a.num_blocks - 1);
-                const uint8_t* base = a.kv + (int64_t)blk * a.kv_bs;
-                b[kt] = fp8_operand(base + (int64_t)slot * kIdxDim, g);
-                ksc[kt] = *reinterpret_cast<const float*>(base + scale_off + 4 * slot);
-            } else {
-                const v8i_t z = {0, 0, 0, 0, 0, 0, 0, 0};
-                b[kt] = z;
-                ksc[kt] = 0.f;
-            }
-        }
-        float p[4];
+        for (int kt = 0; kt < 4; ++kt)  // (positions past the table read its last block: the table index is clamped)
+            blk[s & 1][kt] = bt_row[min(block_of(min(w0 + 256 * s + 16 * kt + c, last)), a.max_blocks - 1)];
+    };
+    look_up(0);
+    look_up(1);
+    v8i_t b[4];
+    float ksc[4], ksc_next[4];
+    auto fetch = [&](int s, int kt) __attribute__((always_inline)) {
+        const int n = min(w0 + 256 * s + 16 * kt + c, last);
+        const int slot = n - block_of(n) * a.block_size;
+        const uint8_t* base = a.kv + (int64_t)min(max(blk[s & 1][kt], 0), a.num_blocks - 1) * a.kv_bs;
+        b[kt] = fp8_operand(base + (int64_t)slot * kIdxDim, g);
+        ksc_next[kt] = *reinterpret_cast<const float*>(base + scale_off + 4 * slot);
+    };
+    constexpr bool kPipe = 16 * HT < kOneQueryHeads;  // (128 heads: no registers for it)
+    if (kPipe) {
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt)
-            p[kt] = qr.gated_part(b[kt]);
-        // lane l: position n0 + l (its key tile g's scale sits in lane (c, g)'s ksc[g])
-        float my_ksc = ksc[0];
+            fetch(0, kt);
+    }
 #pragma unroll
-        for (int kt = 1; kt < 4; ++kt)
-            my_ksc = g == kt ? ksc[kt] : my_ksc;
-        const float v = reduce_scatter4(p) * my_ksc;
+    for (int s = 0; s < kSteps; ++s) {
+        const int n0 = w0 + 256 * s;
+        if (n0 >= n_end)
+            break;
+        float v = a.fill;
+        if (n0 < ctx) {  // (wave-uniform, as is n0)
+            const bool more = kPipe && s + 1 < kSteps && n0 + 256 < ctx;
+            if (!kPipe) {
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt)
+                    fetch(s, kt);
+            }
+            if (s + 2 < kSteps)
+                look_up(s + 2);  // (over step s's entries, which its fetches have read)
+            float p[4];
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt)
+                ksc[kt] = ksc_next[kt];
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) {
+                p[kt] = qr.gated_part(b[kt]);
+                if (more)
+                    fetch(s + 1, kt);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // lane l: position n0 + l (its key tile g's scale sits in lane (c, g)'s ksc[g])
+            float my_ksc = ksc[0];
+#pragma unroll
+            for (int kt = 1; kt < 4; ++kt)
+                my_ksc = g == kt ? ksc[kt] : my_ksc;
+            v = reduce_scatter4(p) * my_ksc;
+        }
         const int n = n0 + lane;
         if (n < n_end)
             out[n] = n < ctx ? v : a.fill;
@@ -391,6 +426,18 @@ void launch_dense(bool small, dim3 grid, hipStream_t st, const MqaArgs& a) {
         hipLaunchKernelGGL((mqa_logits_kernel<FP4, HT, 1, 4>), grid, dim3(kThreadsM), 0, st, a);
     else
         hipLaunchKernelGGL((mqa_logits_kernel<FP4, HT, 2, 4>), grid, dim3(kThreadsM), 0, st, a);
+}
+
+template <int HT>
+void launch_paged(bool fp4, bool shift, dim3 grid, hipStream_t st, const PagedArgs& a) {
+    if (fp4 && shift)
+        hipLaunchKernelGGL((paged_mqa_logits_kernel<true, HT, true>), grid, dim3(kThreadsM), 0, st, a);
+    else if (fp4)
+        hipLaunchKernelGGL((paged_mqa_logits_kernel<true, HT, false>), grid, dim3(kThreadsM), 0, st, a);
+    else if (shift)
+        hipLaunchKernelGGL((paged_mqa_logits_kernel<false, HT, true>), grid, dim3(kThreadsM), 0, st, a);
+    else
+        hipLaunchKernelGGL((paged_mqa_logits_kernel<false, HT, false>), grid, dim3(kThreadsM), 0, st, a);
 }
 
 int check_h(int64_t h) {
@@ -522,28 +569,18 @@ extern "C" int fgv_fp8_fp4_paged_mqa_logits(
     a.block_size = (int32_t)block_size;
     a.max_blocks = (int32_t)max_blocks_per_seq;
     a.max_model_len = (int32_t)max_model_len;
-    a.keys_per_block = 1024;
+    const bool shift = (block_size & (block_size - 1)) == 0;
+    a.block_shift = shift ? __builtin_ctzll((uint64_t)block_size) : 0;
     a.vec_fill = aligned(logits, 16) && logits_stride_row % 4 == 0 && max_model_len % 4 == 0;
     a.fill = clean_logits ? -__builtin_inff() : 0.f;
     const bool fp4 = q_scale != nullptr;
-    const dim3 grid((uint32_t)((max_model_len + a.keys_per_block - 1) / a.keys_per_block), (uint32_t)rows);
+    const dim3 grid((uint32_t)((max_model_len + kPagedKeys - 1) / kPagedKeys), (uint32_t)rows);
     hipStream_t st = static_cast<hipStream_t>(stream);
-#define FGV_PAGED_LAUNCH(FP4, HT) \
-    hipLaunchKernelGGL((paged_mqa_logits_kernel<FP4, HT>), grid, dim3(kThreadsM), 0, st, a)
-#define FGV_PAGED_HEADS(HT)             \
-    do {                                \
-        if (fp4)                        \
-            FGV_PAGED_LAUNCH(true, HT);  \
-        else                            \
-            FGV_PAGED_LAUNCH(false, HT); \
-    } while (0)
     switch (num_heads) {
-        case 16: FGV_PAGED_HEADS(1); break;
-        case 32: FGV_PAGED_HEADS(2); break;
-        case 64: FGV_PAGED_HEADS(4); break;
-        default: FGV_PAGED_HEADS(8); break;
+        case 16: launch_paged<1>(fp4, shift, grid, st, a); break;
+        case 32: launch_paged<2>(fp4, shift, grid, st, a); break;
+        case 64: launch_paged<4>(fp4, shift, grid, st, a); break;
+        default: launch_paged<8>(fp4, shift, grid, st, a); break;
     }
-#undef FGV_PAGED_HEADS
-#undef FGV_PAGED_LAUNCH
     return launch_status();
 }

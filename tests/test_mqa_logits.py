@@ -428,6 +428,19 @@ def test_gpu_paged_edge_cases(fp4):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("block_size", [64, 48, 4])
+@pytest.mark.parametrize("fp4", [False, True])
+def test_gpu_paged_step_edges(fp4, block_size):
+    """Contexts either side of a key tile (16), a wave's step (64), the
+    workgroup's step (256) and its positions (1024), over blocks whose size is
+    a power of two (shifts) or not (divisions)."""
+    _say(f"paged mqa logits step edges fp4={fp4} block_size={block_size}")
+    ctx = torch.tensor([1, 15, 17, 63, 64, 65, 255, 257, 769, 1023, 1024, 1025, 1300, 2047, 2049], dtype=torch.int32)
+    q, cache, w, _, bt = W.make_paged_mqa_inputs(15, 1, 1700, fp4=fp4, block_size=block_size, seed=19)
+    _check_paged(q, cache, w, ctx, bt, 2304, False, rows=torch.arange(15))
+
+
+@pytest.mark.gpu
 def test_gpu_pipeline_from_indexer_ops():
     """The DeepSeek-V4 indexer chain on the GPU: fused_indexer_q_rope_quant
     (FP8 and MXFP4 q, folded weights) -> indexer_k_quant_and_cache (keys into
