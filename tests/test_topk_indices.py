@@ -324,3 +324,26 @@ def test_gpu_combine_rows_past_the_tensor_untouched():
     torch.cuda.synchronize()
     assert torch.equal(comb.cpu()[:T], exp) and torch.equal(lens.cpu()[:T], exp_lens)
     assert bool((comb.cpu()[T:] == -7).all()) and bool((lens.cpu()[T:] == -7).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("topk", [1, 63, 65, 511, 512, 513, 1100])
+def test_gpu_rows_around_a_pass(topk):
+    """Rows shorter and longer than the 512 columns a wave has in flight, both
+    ops, indices past the block table among them."""
+    import flaggems_vllm
+
+    print(f"\n[case] index rows topk={topk}", flush=True)
+    g = torch.Generator().manual_seed(topk)
+    T, blocks = 9, 20
+    loc = torch.randint(-1, 64 * (blocks + 3), (T, topk), generator=g, dtype=I32)
+    req = torch.randint(0, 3, (T,), generator=g, dtype=I32)
+    bt = torch.randint(0, 1000, (3, blocks), generator=g, dtype=I32)
+    exp, exp_lens = oracle.compute_global_topk_indices_and_lens(loc, req, bt, 64)
+    got, lens = flaggems_vllm.compute_global_topk_indices_and_lens(loc.to(DEV), req.to(DEV), bt.to(DEV), 64)
+    assert torch.equal(got.cpu(), exp) and torch.equal(lens.cpu(), exp_lens)
+
+    args = (_t([0, 4, 9]), _t([40, 5000]), _t([40, 300]), 130, 4, topk, 7000, 3000)
+    exp, exp_lens = oracle.combine_topk_swa_indices(loc, *args)
+    got, lens = flaggems_vllm.combine_topk_swa_indices(loc.to(DEV), *(a.to(DEV) if torch.is_tensor(a) else a for a in args))
+    assert torch.equal(got.cpu(), exp) and torch.equal(lens.cpu(), exp_lens)
