@@ -26,8 +26,9 @@
 //     weights) streams from HBM once, x is re-read from L2;
 //   - tiled (larger b): 256 x 128 (or 128 x 128) output tiles over eight
 //     (four) waves of 64 x 64, the K blocks' x and y tiles streamed through a
-//     three-stage LDS ring by LDS DMA, two blocks ahead of the MFMAs (one
-//     workgroup of eight waves per CU).
+//     three-stage LDS ring by LDS DMA and each block's operands read into
+//     registers a block ahead of its MFMAs (one workgroup of eight waves per
+//     CU).
 // The result depends only on the inputs: a fixed K-block order per wave and
 // a fixed order over waves.
 #include "fgv_device.h"
@@ -80,13 +81,6 @@ __device__ __forceinline__ v8i_t load_frag(const uint8_t* row, int g) {
         __builtin_memcpy(&lo, row + 16 * g, 16);
         __builtin_memcpy(&hi, row + 64 + 16 * g, 16);
     }
-    const v8i_t v = {(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-    return v;
-}
-
-__device__ __forceinline__ v8i_t lds_frag(const uint8_t* row, int g) {
-    const uint4 lo = *reinterpret_cast<const uint4*>(row + 16 * g);
-    const uint4 hi = *reinterpret_cast<const uint4*>(row + 64 + 16 * g);
     const v8i_t v = {(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
     return v;
 }
@@ -263,11 +257,20 @@ __global__ void __launch_bounds__(64 * KS) fp8_einsum_skinny_kernel(EinsumArgs a
 // columns over 2 MW waves (64 x 64 each, MW along rows, 2 along columns); x
 // and y rows 16-byte aligned, r > 0.  The K blocks stream through a ring of
 // NS LDS stages by LDS DMA (global_load_lds_dwordx4: each wave
-// instruction lands 64 lanes x 16 bytes = 8 rows contiguously), issued NS - 1
+// instruction lands 64 lanes x 16 bytes = 8 rows contiguously), issued NS
 // blocks ahead of the MFMAs.  Rows are stored unpadded with their 16-byte
 // chunks swizzled, chunk c of row r at (c ^ ((r >> 1) & 7)), so that the 16
 // rows of a fragment read hit 16 distinct chunk slots.  Rows of x past b read
 // row b - 1: they only feed outputs that are not stored.
+//
+// The operands of a block are read into registers during the block before it,
+// between that block's MFMAs, so a block's stage is free as soon as its own
+// MFMAs begin and three blocks are in flight or landed behind it.  (Before,
+// every block read its operands after the barrier, with two blocks behind it:
+// graph replays with the inverse-RoPE quantisation before it, us, h 8, r 4096:
+// b 700 91.2 -> 73.9, b 8192 465 -> 460; h 16, r 7168: b 200, split, 82.5 ->
+// 69.5, b 2500 514 -> 506.  B's and the scales' operands in a second register
+// set spill the 256-row kernel: 1457 us at b 8192.)
 constexpr int kStages4 = 3;  // LDS stages of the 256-row tiles (49 KB each)
 constexpr int kStages2 = 3;  // LDS stages of the 128-row tiles (33 KB each)
 
@@ -310,13 +313,8 @@ struct TileShape {
 template <int MW, int NS, int OUT>
 __global__ void __launch_bounds__(128 * MW) fp8_einsum_tile_kernel(EinsumArgs a, int32_t mtiles, float* part) {
     using S = TileShape<MW>;
-    static_assert(NS >= 2 && NS <= 4, "two to four stages");
-    // the NS stages, named statically by each step of the NS-unrolled loop
-    __shared__ __attribute__((aligned(1024))) uint8_t st0[S::kStageBytes];
-    __shared__ __attribute__((aligned(1024))) uint8_t st1[S::kStageBytes];
-    __shared__ __attribute__((aligned(1024))) uint8_t st2[NS > 2 ? S::kStageBytes : 16];
-    __shared__ __attribute__((aligned(1024))) uint8_t st3[NS > 3 ? S::kStageBytes : 16];
-    auto stage = [&](int i) -> uint8_t* { return i == 0 ? st0 : i == 1 ? st1 : i == 2 ? st2 : st3; };
+    static_assert(NS >= 3, "a block read, one landing, one being sent");
+    __shared__ __attribute__((aligned(1024))) uint8_t st[NS][S::kStageBytes];
 
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -346,22 +344,32 @@ __global__ void __launch_bounds__(128 * MW) fp8_einsum_tile_kernel(EinsumArgs a,
     }
     const float* xsrc = a.xs + (int64_t)hh * a.xs_sh + (int64_t)min(m0 + 64 * wave + lane, a.b - 1) * a.xs_sb;
     const float* ysg = a.ys + (int64_t)hh * a.ys_sh + (int64_t)nt * a.ys_sn;
-    // this wave's DMAs per block (the waitcnt operand while the next block flies)
+    // waves with a scale DMA
     const bool xw = wave < S::kXInstr, yw = wave == S::kYWave;
 
-    auto issue = [&](int kb, uint8_t* st) {
+    // DMA i of this wave's for block kb: x, y rows, then the scales
+    constexpr int kPer = S::kAInstr + S::kBInstr;
+    constexpr int kEvery = kPer < 8 ? 2 : 1;  // MFMAs per DMA
+    auto issue = [&](int kb, uint32_t base, int i) __attribute__((always_inline)) {
         const int64_t k0 = (int64_t)kb * kBlockK;
-        const uint32_t base = lds_addr(st);
-#pragma unroll
-        for (int j = 0; j < S::kAInstr; ++j)
-            dma16(asrc[j] + k0, base + 1024 * (wave * S::kAInstr + j));
-#pragma unroll
-        for (int j = 0; j < S::kBInstr; ++j)
-            dma16(bsrc[j] + k0, base + S::kABytes + 1024 * (wave * S::kBInstr + j));
-        if (xw)
+        if (i < S::kAInstr) {
+            dma16(asrc[i] + k0, base + 1024 * (wave * S::kAInstr + i));
+        } else if (i < kPer) {
+            dma16(bsrc[i - S::kAInstr] + k0, base + S::kABytes + 1024 * (wave * S::kBInstr + i - S::kAInstr));
+        } else if (xw) {
             dma4(xsrc + (int64_t)kb * a.xs_sk, base + S::kXOff + 256 * wave);
-        if (yw)
+        } else if (yw) {
             dma4(ysg + (int64_t)kb * a.ys_sk, base + S::kYOff);
+        }
+    };
+    // waits until at most `blocks` of this wave's blocks are in flight
+    auto wait_blocks = [&](bool one) {
+        if (!one)
+            __builtin_amdgcn_s_waitcnt(wait_vm(0));
+        else if (xw || yw)
+            __builtin_amdgcn_s_waitcnt(wait_vm(kPer + 1));
+        else
+            __builtin_amdgcn_s_waitcnt(wait_vm(kPer));
     };
 
     v4f_t acc[4][4];
@@ -371,77 +379,107 @@ __global__ void __launch_bounds__(128 * MW) fp8_einsum_tile_kernel(EinsumArgs a,
         for (int j = 0; j < 4; ++j)
             acc[i][j] = v4f_t{0.f, 0.f, 0.f, 0.f};
 
-    // one K block: wait for this wave's DMAs of block kb (the next blocks'
-    // may still fly), barrier (everyone's landed; the stage read in the
-    // previous step is free), send block kb + NS - 1 into it, then the MFMAs
-    // on `cur`
-    constexpr int kPer = S::kAInstr + S::kBInstr;  // this wave's DMAs per block (+ 1 with a scale DMA)
-    auto step = [&](int kb, const uint8_t* cur, uint8_t* nxt) {
-        const int after = min(NS - 2, kb_hi - 1 - kb);  // blocks issued after kb
-        if (after >= 2) {
+    // a block's operands in registers
+    v8i_t A[4], B[4];
+    float4 X[4];
+    float Y;
+    const int arow = wm * 64 + c, brow = wn * 64 + c;  // (16 i more keep the swizzle)
+    const uint32_t alo = arow * kBlockK + 16 * swz(arow, g), ahi = arow * kBlockK + 16 * swz(arow, 4 + g);
+    const uint32_t blo = S::kABytes + brow * kBlockK + 16 * swz(brow, g), bhi = S::kABytes + brow * kBlockK + 16 * swz(brow, 4 + g);
+    auto frag = [&](const uint8_t* lo, const uint8_t* hi) __attribute__((always_inline)) {
+        const uint4 l = *reinterpret_cast<const uint4*>(lo), h = *reinterpret_cast<const uint4*>(hi);
+        return v8i_t{(int)l.x, (int)l.y, (int)l.z, (int)l.w, (int)h.x, (int)h.y, (int)h.z, (int)h.w};
+    };
+    auto read_a = [&](const uint8_t* cur, int i) __attribute__((always_inline)) {
+        A[i] = frag(cur + alo + 16 * i * kBlockK, cur + ahi + 16 * i * kBlockK);
+    };
+    auto read_b = [&](const uint8_t* cur, int j) __attribute__((always_inline)) {
+        B[j] = frag(cur + blo + 16 * j * kBlockK, cur + bhi + 16 * j * kBlockK);
+    };
+    auto read_x = [&](const uint8_t* cur, int i) __attribute__((always_inline)) {
+        X[i] = *reinterpret_cast<const float4*>(cur + S::kXOff + 4 * (wm * 64 + 16 * i + 4 * g));
+    };
+    auto read_y = [&](const uint8_t* cur) __attribute__((always_inline)) {
+        Y = reinterpret_cast<const float*>(cur + S::kYOff)[lane];
+    };
+
+    // One K block kb, whose operands are in registers: wait for this wave's
+    // DMAs of block kb + 1, barrier (everyone's landed, and everyone has read
+    // block kb out of its stage), then its MFMAs, with the DMAs of block
+    // kb + 3 - into block kb's stage - and the LDS reads of block kb + 1's
+    // operands between them, each operand after its last use.  A product is
+    // scaled into the accumulator two MFMAs later.
+    auto step = [&](int kb, int at) __attribute__((always_inline)) {
+        const bool next = kb + 1 < kb_hi, send = kb + NS < kb_hi;
+        const uint8_t* nxt = st[at + 1 < NS ? at + 1 : 0];
+        const uint32_t dst = lds_addr(st[at]);
+        if (next) {
+            wait_blocks(kb + 2 < kb_hi);
+            lds_barrier();
+        }
+        v4f_t p[3], sx[2];
+        float y = Y;
+        auto scale_in = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                acc[u >> 2][u & 3][q] = fmaf(p[u % 3][q], sx[(u >> 2) & 1][q], acc[u >> 2][u & 3][q]);
+        };
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int i = u >> 2, j = u & 3;
+            p[u % 3] = mfma_fp8(A[i], B[j]);
+            if (j == 0)
+                sx[i & 1] = v4f_t{X[i].x * y, X[i].y * y, X[i].z * y, X[i].w * y};
+            if (send && u % kEvery == kEvery - 1 && u / kEvery <= kPer)
+                issue(kb + NS, dst, u / kEvery);
+            // (after the last block these read a stage's old bytes, unused)
+            if (j == 3) {
+                read_a(nxt, i);
+                read_x(nxt, i);
+            }
+            if (i == 3)
+                read_b(nxt, j);
+            if (u == 2)
+                read_y(nxt);
+            if (u >= 2)
+                scale_in(u - 2);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        scale_in(14);
+        scale_in(15);
+    };
+    static_assert(16 / kEvery > kPer, "every DMA finds its MFMA");
+
+#pragma unroll
+    for (int j = 0; j < NS; ++j)
+        if (kb_lo + j < kb_hi) {
+#pragma unroll
+            for (int i = 0; i <= kPer; ++i)
+                issue(kb_lo + j, lds_addr(st[j]), i);
+        }
+    if (kb_lo < kb_hi) {
+        // (block kb_lo's DMAs are the oldest: the NS - 1 = 2 blocks behind it may fly)
+        if (kb_lo + 2 < kb_hi) {
             if (xw || yw)
                 __builtin_amdgcn_s_waitcnt(wait_vm(2 * (kPer + 1)));
             else
                 __builtin_amdgcn_s_waitcnt(wait_vm(2 * kPer));
-        } else if (after == 1) {
-            if (xw || yw)
-                __builtin_amdgcn_s_waitcnt(wait_vm(kPer + 1));
-            else
-                __builtin_amdgcn_s_waitcnt(wait_vm(kPer));
         } else {
-            __builtin_amdgcn_s_waitcnt(wait_vm(0));
+            wait_blocks(kb_lo + 1 < kb_hi);
         }
         lds_barrier();
-        if (kb + NS - 1 < kb_hi)
-            issue(kb + NS - 1, nxt);
-        const float sy = reinterpret_cast<const float*>(cur + S::kYOff)[lane];
-        v8i_t A[4], B[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int row = wm * 64 + 16 * i + c;
-            const uint8_t* rp = cur + row * kBlockK;
-            const uint4 lo = *reinterpret_cast<const uint4*>(rp + 16 * swz(row, g));
-            const uint4 hi = *reinterpret_cast<const uint4*>(rp + 16 * swz(row, 4 + g));
-            A[i] = v8i_t{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+            read_a(st[0], i);
+            read_b(st[0], i);
+            read_x(st[0], i);
         }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int row = wn * 64 + 16 * j + c;
-            const uint8_t* rp = cur + S::kABytes + row * kBlockK;
-            const uint4 lo = *reinterpret_cast<const uint4*>(rp + 16 * swz(row, g));
-            const uint4 hi = *reinterpret_cast<const uint4*>(rp + 16 * swz(row, 4 + g));
-            B[j] = v8i_t{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-        }
-        const float* xst = reinterpret_cast<const float*>(cur + S::kXOff);
-        float sx[4][4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float4 v = *reinterpret_cast<const float4*>(xst + wm * 64 + 16 * i + 4 * g);
-            sx[i][0] = v.x * sy;
-            sx[i][1] = v.y * sy;
-            sx[i][2] = v.z * sy;
-            sx[i][3] = v.w * sy;
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const v4f_t p = mfma_fp8(A[i], B[j]);
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    acc[i][j][q] = fmaf(p[q], sx[i][q], acc[i][j][q]);
-            }
-    };
-
-#pragma unroll
-    for (int j = 0; j < NS - 1; ++j)
-        if (kb_lo + j < kb_hi)
-            issue(kb_lo + j, stage(j));
-    for (int kb0 = kb_lo; kb0 < kb_hi; kb0 += NS) {
-#pragma unroll
-        for (int j = 0; j < NS; ++j)
-            if (kb0 + j < kb_hi)
-                step(kb0 + j, stage(j), stage((j + NS - 1) % NS));
+        read_y(st[0]);
+    }
+    int at = 0;
+    for (int kb = kb_lo; kb < kb_hi; ++kb) {
+        step(kb, at);
+        at = at + 1 < NS ? at + 1 : 0;
     }
 
     if (gridDim.z > 1) {
