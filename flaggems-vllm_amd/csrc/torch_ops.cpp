@@ -3,9 +3,9 @@
 //     src/flaggems_vllm/ops/fused_deepseek_v4_qnorm_rope_kv_rope_quant_insert.py:289-351)
 //   fused_inv_rope_fp8_quant                            (reference wrapper
 //     src/flaggems_vllm/ops/fused_inv_rope_fp8_quant.py:157-256)
-// and of the four ops beside them (fused_q_kv_rmsnorm,
+// and of the five ops beside them (fused_q_kv_rmsnorm,
 // dequantize_and_gather_k_cache, fused_indexer_q_rope_quant,
-// compute_slot_mapping_parallel).
+// compute_slot_mapping_parallel, indexer_k_quant_and_cache).
 //
 // The argument checks, the output allocation and the launch run here in C++,
 // so an eager call costs a few microseconds of host time instead of the
@@ -18,7 +18,7 @@
 //   - the dispatcher ops torch.ops.flaggems_vllm.<name> (TORCH_LIBRARY_FRAGMENT;
 //     schemas mark q and k_cache written), for torch.compile and graph capture.
 //     These raise RuntimeError on any failure, as vLLM's own compiled op does.
-// The other four are module functions only; their torch.ops registrations
+// The other five are module functions only; their torch.ops registrations
 // call the Python drop-ins.
 // Launches go on torch's current HIP stream of the tensors' device; nothing
 // synchronises and nothing is read back from the device.
@@ -326,6 +326,36 @@ int indexer_q_rope_quant(const at::Tensor& positions_in, const at::Tensor& index
         scale.defined() ? scale.stride(0) : 0, scale.defined() ? scale.stride(1) : 0, current_stream(index_q));
 }
 
+// indexer_k_quant_and_cache's checks (the ValueError on head_dim stays with
+// the Python drop-in) and launch.  kv_cache[0] and slot_mapping.shape[0]
+// raise IndexError where they do not exist, as there.
+int indexer_k_quant(const at::Tensor& k, const at::Tensor& kv_cache, const at::Tensor& slot_mapping,
+                    int64_t quant_block_size, bool use_ue8m0) {
+    TORCH_CHECK_INDEX(slot_mapping.dim() > 0, "slot_mapping must have a dimension");
+    const int64_t num_tokens = slot_mapping.size(0), head_dim = k.size(-1);
+    FGV_ASSERT(k.scalar_type() == at::kBFloat16 || k.scalar_type() == at::kHalf, "k must be bfloat16 or float16");
+    FGV_ASSERT(kv_cache.dim() == 3 && kv_cache.element_size() == 1,
+               "kv_cache must be [num_blocks, block_size, bytes per token] of a 1-byte type");
+    TORCH_CHECK_INDEX(kv_cache.size(0) > 0, "kv_cache has no block");
+    FGV_ASSERT(blocks_contiguous(kv_cache), "each kv_cache block must be contiguous bytes");
+    FGV_ASSERT(slot_mapping.dim() == 1 && slot_mapping.scalar_type() == at::kLong, "slot_mapping must be 1-D int64");
+    FGV_ASSERT(slot_mapping.stride(0) == 1 || num_tokens <= 1, "slot_mapping must be contiguous");
+    const at::Tensor k2 = k.dim() != 2 ? k.reshape({-1, head_dim}) : k;
+    FGV_ASSERT(k2.size(0) >= num_tokens, "k has fewer rows than slot_mapping");
+    FGV_ASSERT(k2.stride(-1) == 1, "k rows must be contiguous");
+    FGV_ASSERT(kv_cache.device() == k.device() && slot_mapping.device() == k.device(),
+               "all tensors must be on k's device");
+    FGV_ASSERT(k.is_cuda(), "flaggems_vllm runs on the GPU (HIP) only");
+    if (num_tokens == 0)
+        return 0;
+    const c10::DeviceGuard guard(k.device());
+    return fgv_indexer_k_quant_and_cache(k2.data_ptr(), k2.stride(0), k.scalar_type() == at::kHalf ? 1 : 0, num_tokens,
+                                         head_dim, quant_block_size, kv_cache.data_ptr(), kv_cache.stride(0),
+                                         kv_cache.size(0), kv_cache.size(1), slot_mapping.data_ptr<int64_t>(),
+                                         use_ue8m0 ? 1 : 0, current_stream(k));
+}
+
+
 // compute_slot_mapping_parallel (reference
 // src/flaggems_vllm/runtime/backend/_ascend/ops/slot_mapping.py:109-144):
 // slot_mapping written in place.
@@ -403,7 +433,7 @@ TORCH_LIBRARY_IMPL(flaggems_vllm, CUDA, m) {
 
 PYBIND11_MODULE(_fgv_torch, m) {
     m.doc() = "C++ checks and launches of fused_deepseek_v4_qnorm_rope_kv_rope_quant_insert, "
-              "fused_inv_rope_fp8_quant and the four ops beside them (status-returning; the Python drop-ins map "
+              "fused_inv_rope_fp8_quant and the five ops beside them (status-returning; the Python drop-ins map "
               "the status)";
     m.attr("ASSERT_FAILED") = kAssertFailed;
     m.def("qnorm_rope_kv_insert", &qnorm_rope_kv_insert);
@@ -434,5 +464,6 @@ PYBIND11_MODULE(_fgv_torch, m) {
               return std::make_tuple(rc, std::get<0>(out), std::get<1>(out), std::get<2>(out));
           });
     m.def("slot_mapping", &slot_mapping);
+    m.def("indexer_k_quant", &indexer_k_quant);
     m.def("assert_message", []() { return g_assert_message; });
 }

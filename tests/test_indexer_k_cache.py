@@ -665,3 +665,28 @@ def test_gpu_torch_ops_match_functions():
     torch.cuda.synchronize()
     assert torch.equal(a, b)
     assert torch.equal(k1.view(torch.uint8), k2.view(torch.uint8)) and torch.equal(s1, s2)
+
+
+@pytest.mark.parametrize("bad,exc", [
+    (dict(k=torch.zeros(4, 128)), AssertionError),                                          # float32 keys
+    (dict(kv_cache=torch.zeros(2, 16 * 132, dtype=torch.uint8)), AssertionError),          # not 3-D
+    (dict(kv_cache=torch.zeros(2, 16, 132)), AssertionError),                              # 4-byte elements
+    (dict(kv_cache=torch.zeros(0, 16, 132, dtype=torch.uint8)), IndexError),               # no block
+    (dict(kv_cache=torch.zeros(2, 16, 264, dtype=torch.uint8)[..., ::2]), AssertionError),  # block not contiguous
+    (dict(slot_mapping=torch.zeros(4, dtype=torch.int32)), AssertionError),
+    (dict(slot_mapping=torch.zeros(2, 2, dtype=torch.int64)), AssertionError),
+    (dict(slot_mapping=torch.zeros((), dtype=torch.int64)), IndexError),
+    (dict(slot_mapping=torch.zeros(8, dtype=torch.int64)[::2]), AssertionError),
+    (dict(slot_mapping=torch.zeros(5, dtype=torch.int64)), AssertionError),                # more slots than keys
+    (dict(k=torch.zeros(128, 4, dtype=torch.bfloat16).t()), AssertionError),               # keys not contiguous
+    (dict(k=torch.zeros(4, 100, dtype=torch.bfloat16)), ValueError),                       # head_dim % 128
+    (dict(), AssertionError),                                                              # CPU tensors
+])
+def test_insert_refuses_in_order(bad, exc):
+    import flaggems_vllm
+
+    args = dict(k=torch.zeros(4, 128, dtype=torch.bfloat16), kv_cache=torch.zeros(2, 16, 132, dtype=torch.uint8),
+                slot_mapping=torch.zeros(4, dtype=torch.int64), quant_block_size=128, scale_fmt="ue8m0")
+    args.update(bad)
+    with pytest.raises(exc):
+        flaggems_vllm.indexer_k_quant_and_cache(**args)
