@@ -881,7 +881,7 @@ def main():
         from flaggems_vllm import _native
 
         split = _native.lib().fgv_top_k_per_row_workspace_bytes(R, V, k) > 0
-        kernel = "top_k_part_kernel" if split else "top_k_per_row_kernel"
+        kernel = "top_k_part_kernel" if split else "top_k_row_kernel" if V <= 16384 else "top_k_per_row_kernel"
         workload = f"{args.topk_case}_R{R}_V{V}_k{k}"
         config = {"workload": f"top_k_per_row_{'decode' if args.topk_case == 'decode' else 'prefill'} "
                               f"{R} rows x {V} float32 logits (row stride {s0}), top_k {k}, full rows",

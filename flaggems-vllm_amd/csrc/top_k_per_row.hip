@@ -489,9 +489,9 @@ __device__ __forceinline__ void long_row(const TopkArgs& a, const float* x, int3
     }
 }
 
-// LONG = false: rows of at most CACHE values (the launcher's width), held in
-// LDS.  LONG = true: any row; longer ones are streamed.
-template <int CACHE, int THREADS, bool LONG>
+// Any row: one of at most CACHE values is held in LDS, longer ones are
+// streamed.
+template <int CACHE, int THREADS>
 __global__ void __launch_bounds__(THREADS)
 top_k_per_row_kernel(TopkArgs a) {
     using B = Block<THREADS>;
@@ -506,15 +506,13 @@ top_k_per_row_kernel(TopkArgs a) {
     const int t = threadIdx.x;
     const int32_t r = blockIdx.x;
     int32_t start;
-    int32_t len = row_range(a, r, start);
+    const int32_t len = row_range(a, r, start);
     int32_t* orow = a.out + (int64_t)r * a.os0;
     const int32_t k = a.k;
     if (len <= k) {
         write_short_row<THREADS>(orow, a.os1, len, k);
         return;
     }
-    if (!LONG && len > CACHE)
-        len = CACHE;  // not reached: the launcher keeps width <= CACHE here
     const float* x = a.logits + (int64_t)r * a.s0 + (int64_t)start * a.s1;
     auto clear = [&]() {
         for (int b = t; b < kBins; b += THREADS)
@@ -534,7 +532,7 @@ top_k_per_row_kernel(TopkArgs a) {
     }
     __syncthreads();
 
-    if (!LONG || len <= CACHE) {
+    if (len <= CACHE) {
         // ---- the row in LDS
         for_each<THREADS, kRowDepth>(x, a.s1, len, [&](float v, int32_t i) {
             const uint32_t key = order_key(v);
@@ -545,9 +543,152 @@ top_k_per_row_kernel(TopkArgs a) {
         lds_select<THREADS>(cache, nullptr, len, (uint32_t)k, hist, wsum, sel, emit);
         return;
     }
-    if constexpr (LONG)
-        long_row<CACHE, THREADS>(a, x, len, k, cache, hist, wsum, sel, counters, emit);
+    long_row<CACHE, THREADS>(a, x, len, k, cache, hist, wsum, sel, counters, emit);
 }
+
+// ---- Rows of at most THREADS * N values: the keys in registers, N (and the
+// row's unaligned head and tail) per thread.  Key 0, below every value's, marks
+// a slot past the row.  The three histogram passes and the output pass then
+// read registers, where the row in LDS cost each of them a dependent LDS read
+// per value; LDS holds the histogram only.  Kept values are counted and placed
+// by one scan over the threads, so a row's output order is fixed.  What bounds
+// it: the scans' barriers and the histogram atomics (randn rows crowd into few
+// bins).  Measured against the row in LDS (graph
+// replays, randn rows, k 512, us): 24 x 16384 17.1 -> 14.1, 1024 x 9000 28.1 ->
+// 25.8, 2048 x 16384 79.8 -> 63.5, 64 x 4096 10.2 -> 8.6, 16383 x 4095 143 ->
+// 113, 512 x 9000 15.4 -> 15.9.
+template <int THREADS, int N>
+__device__ __forceinline__ void row_select(const TopkArgs& a, int32_t r, int32_t start, int32_t len, uint32_t* hist,
+                                           uint32_t* wsum, int32_t* sel) {
+    using B = Block<THREADS>;
+    static_assert(THREADS * N <= 8 * kBins, "a row's index is a bin and three bits");
+    const int t = threadIdx.x;
+    int32_t* orow = a.out + (int64_t)r * a.os0;
+    const int32_t k = a.k;
+    const float* x = a.logits + (int64_t)r * a.s0 + (int64_t)start * a.s1;
+    const bool unit = a.s1 == 1;
+    // unit stride: slots 4u..4u+3 are the float4 u * THREADS + t past the head
+    // (h values up to a 16-byte boundary), slot N value t of the head, N + 1 of
+    // the tail; other strides: slot n is value n * THREADS + t
+    const int32_t head = (int32_t)(((16 - ((uintptr_t)x & 15)) & 15) >> 2);
+    const int32_t h = head < len ? head : len, n4 = (len - h) >> 2;
+    uint32_t key[N + 2];
+    auto index = [&](int n) {
+        if (!unit)
+            return n * THREADS + t;
+        return n < N ? h + 4 * ((n >> 2) * THREADS + t) + (n & 3) : n == N ? t : h + 4 * n4 + t;
+    };
+    key[N] = key[N + 1] = 0;
+    if (unit) {
+        // (loads past the last float4 return zero and are not used)
+        const __amdgpu_buffer_rsrc_t rs =
+            __builtin_amdgcn_make_buffer_rsrc((void*)(x + h), (short)0, n4 * 16, kBufferWord3);
+        uint32_t __attribute__((ext_vector_type(4))) q[N / 4];
+#pragma unroll
+        for (int u = 0; u < N / 4; ++u)
+            q[u] = __builtin_amdgcn_raw_buffer_load_b128(rs, t * 16, u * THREADS * 16, 0);
+        if (t < h)
+            key[N] = order_key(x[t]);
+        if (h + 4 * n4 + t < len)
+            key[N + 1] = order_key(x[h + 4 * n4 + t]);
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+            key[n] = (n >> 2) * THREADS + t < n4 ? order_key(__uint_as_float(q[n >> 2][n & 3])) : 0u;
+    } else {
+        float v[N];
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+            v[n] = n * THREADS + t < len ? x[(int64_t)(n * THREADS + t) * a.s1] : 0.f;
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+            key[n] = n * THREADS + t < len ? order_key(v[n]) : 0u;
+    }
+    auto clear = [&]() {
+        for (int b = t; b < kBins; b += THREADS)
+            hist[b] = 0;
+    };
+    // one level: counts bin(n) of the slots that keep(n), and finds the bin of
+    // the need-th largest; leaves need counted within that bin
+    uint32_t need = (uint32_t)k;
+    auto level = [&](auto&& keep, auto&& bin) __attribute__((always_inline)) {
+        clear();
+        __syncthreads();
+#pragma unroll
+        for (int n = 0; n < N + 2; ++n)
+            if (keep(n))
+                atomicAdd(&hist[bin(n)], 1u);
+        __syncthreads();
+        B::find_bin(hist, need, wsum, sel);
+        const uint32_t b = sel[0];
+        need -= sel[1];
+        return b;
+    };
+    const uint32_t b1 = level([&](int n) { return key[n] != 0; }, [&](int n) { return key[n] >> 21; });
+    const uint32_t b2 = level([&](int n) { return key[n] != 0 && key[n] >> 21 == b1; },
+                              [&](int n) { return (key[n] >> 10) & 0x7ff; });
+    const uint32_t p2 = b1 << 11 | b2;
+    const uint32_t b3 = level([&](int n) { return key[n] != 0 && key[n] >> 10 == p2; },
+                              [&](int n) { return key[n] & 0x3ff; });
+    const uint32_t key_t = p2 << 10 | b3;
+    // the values equal to the k-th largest: all of them, or the `need` with the
+    // smallest indices, found as the largest of 8 kBins - 1 - index
+    int32_t last = 0x7fffffff;
+    const uint32_t ties = hist[b3];
+    if (need != ties) {
+        __syncthreads();  // every thread has read `ties`
+        auto rev = [&](int n) { return (uint32_t)(8 * kBins - 1 - index(n)); };
+        const uint32_t c1 = level([&](int n) { return key[n] == key_t; }, [&](int n) { return rev(n) >> 3; });
+        const uint32_t c2 = level([&](int n) { return key[n] == key_t && rev(n) >> 3 == c1; },
+                                  [&](int n) { return rev(n) & 7; });
+        last = 8 * kBins - 1 - (int32_t)(c1 << 3 | c2);
+    }
+    auto kept = [&](int n) { return key[n] > key_t || (key[n] == key_t && index(n) <= last); };
+    uint32_t mine = 0, total;
+#pragma unroll
+    for (int n = 0; n < N + 2; ++n)
+        mine += kept(n) ? 1u : 0u;
+    uint32_t p = B::scan(mine, wsum, total);
+#pragma unroll
+    for (int n = 0; n < N + 2; ++n)
+        if (kept(n)) {
+            orow[(int64_t)p * a.os1] = index(n);
+            ++p;
+        }
+}
+
+// Each row takes the fewest slots, in steps of 4, that hold it: every pass walks
+// all of them.  (With the launch's most for every row, ragged prefill rows of
+// 2400 to 4096 values in 9800 columns ran slower than in LDS; in steps of 8,
+// 512 rows of 9000 17.1 us, 15.4 in LDS.)
+template <int THREADS, int N, int MAXN>
+__device__ __forceinline__ void fewest_slots(const TopkArgs& a, int32_t r, int32_t start, int32_t len, uint32_t* hist,
+                                             uint32_t* wsum, int32_t* sel) {
+    if constexpr (N < MAXN) {
+        if (len > N * THREADS) {
+            fewest_slots<THREADS, N + 4, MAXN>(a, r, start, len, hist, wsum, sel);
+            return;
+        }
+    }
+    row_select<THREADS, N>(a, r, start, len, hist, wsum, sel);
+}
+
+// Rows of at most THREADS * MAXN columns.
+template <int THREADS, int MAXN>
+__global__ void __launch_bounds__(THREADS)
+top_k_row_kernel(TopkArgs a) {
+    __shared__ uint32_t hist[kBins];
+    __shared__ uint32_t wsum[Block<THREADS>::kWaves];
+    __shared__ int32_t sel[2];
+    const int32_t r = blockIdx.x;
+    int32_t start;
+    const int32_t len = row_range(a, r, start);
+    if (len <= a.k) {
+        write_short_row<THREADS>(a.out + (int64_t)r * a.os0, a.os1, len, a.k);
+        return;
+    }
+    fewest_slots<THREADS, 4, MAXN>(a, r, start, len, hist, wsum, sel);
+}
+
 // ---- Rows split into parts: rows longer than the LDS row cache, when the
 // caller's workspace holds every part's candidates.  Part p of a row is
 // [p * cl, min(len, (p + 1) * cl)), cl = ceil(len / parts) <= kPartCache; its
@@ -706,15 +847,15 @@ int launch_topk(TopkArgs a, int64_t num_rows, void* workspace, int64_t workspace
     }
     const dim3 grid((unsigned)num_rows);
     if (a.width <= 4096)
-        hipLaunchKernelGGL((top_k_per_row_kernel<4096, 256, false>), grid, dim3(256), 0, st, a);
+        hipLaunchKernelGGL((top_k_row_kernel<256, 16>), grid, dim3(256), 0, st, a);
     else if (a.width <= 8192)
-        hipLaunchKernelGGL((top_k_per_row_kernel<8192, 512, false>), grid, dim3(512), 0, st, a);
+        hipLaunchKernelGGL((top_k_row_kernel<512, 16>), grid, dim3(512), 0, st, a);
     else if (a.width <= 16384)
-        hipLaunchKernelGGL((top_k_per_row_kernel<16384, 512, false>), grid, dim3(512), 0, st, a);
+        hipLaunchKernelGGL((top_k_row_kernel<512, 32>), grid, dim3(512), 0, st, a);
     else if (num_rows <= cu_count())  // a CU per row: 1024 threads stream it faster
-        hipLaunchKernelGGL((top_k_per_row_kernel<8192, 1024, true>), grid, dim3(1024), 0, st, a);
+        hipLaunchKernelGGL((top_k_per_row_kernel<8192, 1024>), grid, dim3(1024), 0, st, a);
     else  // two rows per CU
-        hipLaunchKernelGGL((top_k_per_row_kernel<12288, 512, true>), grid, dim3(512), 0, st, a);
+        hipLaunchKernelGGL((top_k_per_row_kernel<12288, 512>), grid, dim3(512), 0, st, a);
     return launch_status();
 }
 

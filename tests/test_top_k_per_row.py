@@ -358,3 +358,22 @@ def test_gpu_many_short_rows(k):
     ends[8::50] = V + 5                                          # past the width
     rows = sorted(set(range(0, R, 7)) | set(range(1, 80)) | {R - 1})
     _run_prefill(logits, starts, ends, k, rows)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width", [4096, 8192, 16384])
+def test_gpu_row_slots(width):
+    """Rows in registers: lengths either side of every slot count (4 to 32 in
+    steps of 4) of the three launches, starts at every 4-byte offset from a
+    16-byte boundary, and half the rows with few distinct values, so that ties
+    at the k-th go by index."""
+    threads = 256 if width == 4096 else 512
+    k = 200
+    lens = [n for s in range(4, width // threads + 1, 4) for n in (s * threads - 1, s * threads, s * threads + 1)]
+    lens = [min(n, width) for n in lens] + [k + 1, k, width]
+    g = torch.Generator().manual_seed(width)
+    x = torch.randn(len(lens), width, generator=g)
+    x[1::2] = torch.randint(0, 5, x[1::2].shape, generator=g).float()
+    starts = torch.tensor([min(i % 5, width - n) for i, n in enumerate(lens)], dtype=I32)
+    ends = starts + torch.tensor(lens, dtype=I32)
+    _run_prefill(x, starts, ends, k, range(len(lens)))
