@@ -1060,6 +1060,32 @@ def test_gpu_pieces_against_oracle(case):
         assert torch.allclose(l.double()[fin], l64[fin], rtol=1e-5, atol=1e-5), what
 
 
+@pytest.mark.gpu
+def test_gpu_pieces_graph_replays():
+    """Pieces and merge captured in a HIP graph: every replay, with eager work
+    between, equals the eager call."""
+    import flaggems_vllm
+
+    print("\n[case] sparse MLA pieces graph", flush=True)
+    d, other = _pieces_case("few").to(DEV), _pieces_case("least").to(DEV)
+    call = lambda w: flaggems_vllm.flash_mla_with_kvcache(w.q, w.k_cache, None, None, 512, _meta(), is_fp8_kvcache=True,
+                                                          indices=w.indices, **w.kwargs())
+    ref, ref_lse = (t.clone() for t in call(d))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out, lse = call(d)
+    for i in range(3):
+        out.fill_(7.0)
+        lse.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), ref.view(torch.int16)), f"replay {i}"
+        assert torch.equal(lse, ref_lse), f"replay {i}"
+        call(other)
+        torch.cuda.synchronize()
+
+
 def test_pieces_rule():
     """Where items are cut, and that what the query asks for is bounded."""
     from flaggems_vllm import _native
