@@ -18,8 +18,10 @@
 // histograms in LDS (bits 31..21, 20..10, 9..0), each level counting only the
 // values whose higher bits match the level above and picking the bin that
 // holds the k-th largest:
-//   - rows up to CACHE values are read from HBM once into LDS as keys, and
-//     every level runs over LDS;
+//   - in launches of at most 16384 columns a row's keys are read once into
+//     registers, and every level runs over them (top_k_row_kernel);
+//   - wider launches hold rows up to CACHE values in LDS as keys, and every
+//     level runs over LDS (top_k_per_row_kernel);
 //   - longer rows are read once: an evenly spaced sample of the row (1/32 of
 //     it, at least 2048 values) gives a key that about 4k of the row's values
 //     reach, and one pass keeps every value at or above it, (key, index), in
