@@ -376,6 +376,9 @@ static_assert(kQLoads < 64, "vmcnt holds 6 bits");
 // s_waitcnt operand "lgkmcnt(0)" alone.
 constexpr int kWaitLds = 15 | (3 << 14) | (7 << 4);
 
+// s_waitcnt operand "vmcnt(0)" alone: every global load and LDS DMA of the wave.
+constexpr int kWaitVm = (7 << 4) | (15 << 8);
+
 // Workgroup barrier over LDS work only.  __syncthreads' fence (even one
 // scoped to LDS) waits for every outstanding global load, q's included, since
 // LDS-DMA writes count there too; the callers wait for their LDS-DMA gathers
@@ -1519,6 +1522,9 @@ sparse_mla_decode_pair_kernel(MlaArgs a) {
             if (k + 1 < K)
                 expanded_step(k + 1, kbuf, raw_tile);
         }
+        // The compiler does not know of the lengths' DMAs (lds_len, read below
+        // by every wave), and a half without a chunk has waited for none yet.
+        __builtin_amdgcn_s_waitcnt(kWaitVm);
         __syncthreads();  // both halves done: every K tile and gather buffer is free
 
         // ---- the second item (first pass only): this item's rank among
