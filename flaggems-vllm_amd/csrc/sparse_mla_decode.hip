@@ -575,7 +575,12 @@ __device__ __forceinline__ void run_segment(const MlaArgs& a, uint8_t (&raw)[2][
         const int id_cur = load_id(select(v0, v1, c_lo >= n0), first_of(c_lo), wave, lane);
         if (c_lo + 1 < c_hi)
             id_next = load_id(select(v0, v1, c_lo + 1 >= n0), first_of(c_lo + 1), wave, lane);
+        // (The compiler lays the two branches out one behind the other and takes
+        // the other one's loads for possibly in flight: without the wait, which
+        // costs nothing beside the wait for id_cur, it would wait for them
+        // behind the gather, and so drain the gather before q's loads go out.)
         if (c_lo < c_mid) {
+            __builtin_amdgcn_s_waitcnt(kWaitVm);
             issue_gather(select(v0, v1, c_lo >= n0), dummy, wave, lane, id_cur, raw[c_lo & 1], mask_lds[c_lo & 1]);
             load_q();
         } else {
@@ -604,7 +609,7 @@ __device__ __forceinline__ void run_segment(const MlaArgs& a, uint8_t (&raw)[2][
         attend_chunk(kt, mask, qf, acc, m_run, l_run, qk_base, tr_base, g, a.scale_log2);
     };
 
-    for (int c = c_lo; c < c_mid; ++c) {
+    auto raw_step = [&](int c, bool first) __attribute__((always_inline)) {
         uint8_t* cur = raw[c & 1];
         // The gather and dequantisation addresses derive from the lane id; an
         // opaque copy per chunk keeps them from being held (and spilled)
@@ -613,7 +618,7 @@ __device__ __forceinline__ void run_segment(const MlaArgs& a, uint8_t (&raw)[2][
         asm volatile("" : "+v"(ln));
         // This wave's gathers of chunk c (and chunk c+1's index); on the first
         // chunk, all but q's loads, which are issued last.
-        if (c == c_lo)
+        if (first)
             __builtin_amdgcn_s_waitcnt(kWaitAllButQ);
         else
             __builtin_amdgcn_s_waitcnt(0);
@@ -628,7 +633,20 @@ __device__ __forceinline__ void run_segment(const MlaArgs& a, uint8_t (&raw)[2][
         if (c + 2 < c_hi)
             id_next = load_id(select(v0, v1, c + 2 >= n0), first_of(c + 2), wave, ln);
         attend(kbuf, mask_lds[c & 1]);
-    }
+    };
+    // The first chunk on its own: with its wait in the loop the compiler takes
+    // q's loads and id_next for possibly in flight on every chunk, and waits
+    // for them behind the next gather, which drains the gather too (it does
+    // not count those DMAs).  So measured, against the first chunk's wait in
+    // the loop (extra caches too large to expand, us): split grid, 250 rows of
+    // 128 + 2048 156.5 -> 150, 600 ragged rows 198 -> 189; paired grid (which
+    // keeps its wait in the loop, one copy of the code, and states behind its
+    // dequantisation that nothing is in flight), 300 such rows 241.7 -> 235.5,
+    // 400 ragged 138 -> 135.
+    if (c_lo < c_mid)
+        raw_step(c_lo, true);
+    for (int c = c_lo + 1; c < c_mid; ++c)
+        raw_step(c, false);
     // One expanded chunk: its rows are read from `tile` while the next chunk's
     // rows stream into `other`.  The loop below runs these in (raw, K tile)
     // pairs, so that each step reads one fixed array (two steps under an
@@ -1460,6 +1478,7 @@ sparse_mla_decode_pair_kernel(MlaArgs a) {
             if (K > 1)
                 id_next = load_id(view_of(1), first_of(1), hw, lane);
             if (Kc > 0) {
+                __builtin_amdgcn_s_waitcnt(kWaitVm);  // as in run_segment
                 issue_gather(view_of(0), mla_zero_entry, hw, lane, id_cur, raw[0], mask_lds[0]);
                 load_q();
             } else {
@@ -1495,6 +1514,7 @@ sparse_mla_decode_pair_kernel(MlaArgs a) {
             half_barrier(&lds_hbar[half], gen);  // the half's gathers landed; its K tile no longer read
             dequantize(raw[k & 1], kbuf, hw, ln);
             half_barrier(&lds_hbar[half], gen);
+            __builtin_amdgcn_s_waitcnt(kWaitVm);  // as in run_segment
             if (k + 1 < Kc)
                 issue_gather(view_of(k + 1), mla_zero_entry, hw, ln, id_next, raw[(k + 1) & 1],
                              mask_lds[(k + 1) & 1]);

@@ -36,3 +36,31 @@ def test_pair_kernel_waits_for_its_length_dmas(mla_asm):
     at = next(i for i in range(last, len(code)) if code[i].startswith("s_barrier"))
     before = code[at - 4:at]
     assert any(re.match(r"s_waitcnt\b.*vmcnt\(0\)", line) for line in before), before
+
+
+@pytest.mark.parametrize("kernel", ["decode", "decode_pieces", "decode_split", "decode_pair"])
+def test_no_wait_drains_a_gather(mla_asm, kernel):
+    """Behind a raw gather (its scale words go last), no wait for vector
+    memory before q's loads go out (the first gather), nor before the current
+    chunk's scores, 32 MFMAs, are made (the chunk loops'): either would also
+    wait for the gather, which is meant to land under them.  The gather under
+    the first chunk is left out where that chunk has code of its own (its
+    scores wait for q), and so is the paired kernel's first (its q addresses
+    are reloaded registers)."""
+    code, seen = mla_asm[f"sparse_mla_{kernel}_kernel"], []
+    for i, line in enumerate(code):
+        if not line.startswith("global_load_lds_dword "):
+            continue
+        at = next((j for j in range(i, len(code)) if code[j].startswith(("v_mfma", "global_load_dwordx4"))), None)
+        if at is None:
+            continue
+        first = code[at].startswith("global_load_dwordx4")
+        end = at if first else [j for j in range(at, len(code)) if code[j].startswith("v_mfma")][31]
+        seen.append((first, [x for x in code[i:end] if re.match(r"s_waitcnt\b.*vmcnt", x)]))
+    if kernel == "decode_pair":
+        seen = [s for s in seen if not s[0]]
+        assert len(seen) == 1
+    else:
+        assert [s[0] for s in seen] == [True, False, False]
+        del seen[1]
+    assert not any(waits for _, waits in seen), seen
