@@ -1061,6 +1061,29 @@ def test_gpu_pieces_against_oracle(case):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("batch,chunks", [(8, 4), (24, 5), (100, 10), (128, 19), (224, 32)])
+def test_gpu_pieces_short_rows_whole(batch, chunks):
+    """Rows of at most a chunk more than a piece of the longest possible row
+    are not cut: the bits of the uncut call, with one row among them that is
+    cut."""
+    print(f"\n[case] sparse MLA pieces, short rows batch={batch} chunks={chunks}", flush=True)
+    extra = 1856 if batch == 224 else 1024
+    w = W.make_mla_workload(batch=batch, topk=128, num_pages=16, extra_topk=extra, extra_page=64, extra_pages=500,
+                            seed=97, q_scale=0.1)
+    n = 32 * chunks - torch.arange(batch, dtype=torch.int32) % 32
+    w.topk_length = n.clamp(max=128).to(torch.int32)
+    w.extra_topk_length = (n - w.topk_length).to(torch.int32)
+    w.extra_topk_length[batch // 2] = extra
+    assert _grid(w) == 3
+    out, lse, _ = _gpu_raw(w, workspace=True)
+    uncut, uncut_lse, _ = _gpu_raw(w, workspace=False)
+    rows = torch.arange(batch) != batch // 2
+    assert torch.equal(out[rows].view(torch.int16), uncut[rows].view(torch.int16))
+    assert torch.equal(lse[rows], uncut_lse[rows])
+    assert torch.allclose(lse[~rows], uncut_lse[~rows], rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.gpu
 def test_gpu_pieces_graph_replays():
     """Pieces and merge captured in a HIP graph: every replay, with eager work
     between, equals the eager call."""
@@ -1093,10 +1116,12 @@ def test_pieces_rule():
     f = _native.lib().fgv_sparse_mla_decode_workspace_bytes
     grid = _native.lib().fgv_sparse_mla_decode_grid
     slot = (64 * 512 + 128) * 4
-    assert grid(24, 1, 64, 128, 512) == 3 and f(24, 1, 64, 128, 512, 1 << 20) == 24 * 10 * slot
+    assert grid(24, 1, 64, 128, 512) == 3 and f(24, 1, 64, 128, 512, 1 << 20) == 24 * 5 * slot
     assert grid(24, 1, 64, 256, 0) == 0 and f(24, 1, 64, 256, 0, 0) == 0          # 8 chunks: whole
     assert grid(128, 1, 64, 128, 512) == 3 and grid(129, 1, 64, 128, 512) == 0    # more items than half the CUs
-    assert grid(248, 1, 64, 128, 1024) == 3 and grid(256, 1, 64, 128, 1024) == 0  # long: two pieces each fit
+    # two pieces each fit, but cost more than they give for 36 chunks (79.7 us whole, 84.0 cut), not for 62
+    # (128.0 whole, 118.1 cut); at 256 items they do not fit
+    assert grid(248, 1, 64, 128, 1024) == 0 and grid(248, 1, 64, 128, 1856) == 3 and grid(256, 1, 64, 128, 1856) == 0
     assert grid(100, 1, 64, 128, 192) == 0                                        # not worth the slots
     assert f(24, 1, 64, 128, 512, 1000) == 1000 * 1024                            # expanded: not cut
     for batch in range(1, 257):
