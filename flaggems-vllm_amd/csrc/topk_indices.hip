@@ -28,8 +28,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kRowsPerBlock = kThreads / 64;
-constexpr int kAhead = 8;        // columns a lane has in flight
-constexpr int32_t kNoSlot = -2;  // a local index (counted) whose block the table does not hold
+constexpr int kMostAhead = 8;    // columns a lane has in flight, at most
 
 __device__ __forceinline__ int32_t wrap_mul(int32_t a, int32_t b) { return (int32_t)((uint32_t)a * (uint32_t)b); }
 __device__ __forceinline__ int32_t wrap_add(int32_t a, int32_t b) { return (int32_t)((uint32_t)a + (uint32_t)b); }
@@ -49,6 +48,15 @@ struct GlobalArgs {
     int32_t topk, block_size;
 };
 
+// A row's columns go to a wave in passes of 64 kAhead, a pass's loads in
+// flight together: the row is a chain of two dependent loads per pass, not of
+// two per 64 columns.  The launcher takes as few passes as kMostAhead allows
+// and then the fewest columns per lane that make them: a lane's unused columns
+// are not free (8192 rows of 64 with eight per lane 7.5 us, with one 3.4).
+// Measured with one column per lane / eight / as here, us: 24 rows of 128
+// columns 2.6 / 3.3 / 2.5, of 512 4.5 / 4.1 / 4.0; 8192 rows of 64 3.5 / 7.5 /
+// 3.5, of 512 12.2 / 12.3 / 10.8; 4096 rows of 2048 28.6 / 21.5 / 19.8.
+template <int kAhead>
 __global__ void __launch_bounds__(kThreads)
 global_topk_indices_kernel(GlobalArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -56,34 +64,38 @@ global_topk_indices_kernel(GlobalArgs a) {
     if (t >= a.num_tokens)
         return;
     const int64_t row = (int64_t)a.req[t] * a.table_stride;
-    const int32_t* lrow = a.local + t * a.local_s0;
-    int32_t* orow = a.out + t * a.out_s0;
+    const int32_t* lcol = a.local + t * a.local_s0 + lane * a.local_s1;
+    int32_t* ocol = a.out + t * a.out_s0 + lane * a.out_s1;
+    const int64_t lstep = 64 * a.local_s1, ostep = 64 * a.out_s1;
     int32_t count = 0;
-    // kAhead columns per lane at a time, their loads in flight together: the
-    // row is a chain of two dependent loads, not of two per 64 columns (24 rows
-    // of 512: 7.1 -> 4.5 us)
-    for (int32_t i0 = lane; i0 - lane < a.topk; i0 += 64 * kAhead) {
+    // (unsigned: the last pass of a row near 2^31 columns ends past them)
+    const uint32_t topk = (uint32_t)a.topk;
+    for (uint32_t i0 = lane; i0 - lane < topk; i0 += 64 * kAhead) {
         int32_t l[kAhead], b[kAhead];
 #pragma unroll
         for (int k = 0; k < kAhead; ++k)
-            l[k] = i0 + 64 * k < a.topk ? lrow[(i0 + 64 * k) * a.local_s1] : -1;
+            l[k] = i0 + 64 * k < topk ? lcol[k * lstep] : -1;
 #pragma unroll
         for (int k = 0; k < kAhead; ++k) {
             // a block outside the table (an invalid local index or request)
             // has no slot; the reference would read past its row
-            const int64_t f = row + l[k] / a.block_size;
-            b[k] = -1;
-            if (l[k] >= 0 && f >= 0 && f < a.table_span)
+            const int32_t blk = l[k] / a.block_size;
+            const int64_t f = row + blk;
+            count += __popcll(__ballot(l[k] >= 0));
+            b[k] = 0;
+            if (l[k] >= 0 && f >= 0 && f < a.table_span) {
                 b[k] = a.table[f];
-            else
-                l[k] = l[k] >= 0 ? kNoSlot : -1;
-            count += __popcll(__ballot(l[k] != -1));
+                l[k] -= blk * a.block_size;
+            } else {
+                l[k] = -1;
+            }
         }
 #pragma unroll
         for (int k = 0; k < kAhead; ++k)
-            if (i0 + 64 * k < a.topk)
-                orow[(i0 + 64 * k) * a.out_s1] =
-                    l[k] < 0 ? -1 : wrap_add(wrap_mul(b[k], a.block_size), l[k] - l[k] / a.block_size * a.block_size);
+            if (i0 + 64 * k < topk)
+                ocol[k * ostep] = l[k] < 0 ? -1 : wrap_add(wrap_mul(b[k], a.block_size), l[k]);
+        lcol += kAhead * lstep;
+        ocol += kAhead * ostep;
     }
     if (lane == 0)
         a.lens[t] = (a.valid == nullptr || a.valid[t] != 0) ? count : 0;
@@ -107,6 +119,12 @@ struct CombineArgs {
 // over a request's tokens.  Tokens outside every request are not written, and
 // neither are tokens that query_start_loc places outside [0, num_tokens) (the
 // tensors' rows), which the reference would read and write out of bounds.
+// Columns per lane and pass as in the kernel above (by the row width).
+// Measured with one column per lane / eight / as here, us, top-k and a window
+// of 128: 24 rows of 128 2.6 / 3.0 / 2.6, of 512 3.7 / 3.8 / 3.3; 8192 rows of
+// 64 5.7 / 7.4 / 5.9, of 512 17.8 / 14.1 / 12.9; 4096 rows of 2048 30.3 / 18.1 /
+// 17.6.
+template <int kAhead>
 __global__ void __launch_bounds__(kThreads)
 combine_topk_swa_kernel(CombineArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -126,31 +144,52 @@ combine_topk_swa_kernel(CombineArgs a) {
         const int32_t topk_len = min((pos + 1) / a.ratio, a.topk_n);
         const int32_t swa_len = min(pos + 1, a.window);
         const int32_t swa_base = wrap_add(wrap_add(row_off, a.n), pos - swa_len + 1 - gather_start);
-        const int32_t* trow = a.topk + (int64_t)t * a.topk_s0;
-        int32_t* orow = a.out + (int64_t)t * a.out_s0;
-        for (int32_t c0 = lane; c0 - lane < a.width; c0 += 64 * kAhead) {
+        const int32_t* tcol = a.topk + (int64_t)t * a.topk_s0 + lane * a.topk_s1;
+        int32_t* ocol = a.out + (int64_t)t * a.out_s0 + lane * a.out_s1;
+        const int64_t tstep = 64 * a.topk_s1, ostep = 64 * a.out_s1;
+        const uint32_t width = (uint32_t)a.width, topk_cols = (uint32_t)max(topk_len, 0);
+        for (uint32_t c0 = lane; c0 - lane < width; c0 += 64 * kAhead) {
             int32_t v[kAhead];
 #pragma unroll
             for (int k = 0; k < kAhead; ++k) {
-                const int32_t c = c0 + 64 * k;
+                const uint32_t c = c0 + 64 * k;
                 v[k] = 0;
-                if (c < topk_len)
-                    v[k] = trow[c * a.topk_s1];
+                if (c < topk_cols)
+                    v[k] = tcol[k * tstep];
             }
 #pragma unroll
             for (int k = 0; k < kAhead; ++k) {
-                const int32_t c = c0 + 64 * k;
+                const uint32_t c = c0 + 64 * k;
+                const int32_t w = (int32_t)c - topk_len;
                 int32_t x = -1;
-                if (c < topk_len)
+                if (c < topk_cols)
                     x = wrap_add(v[k], row_off);
-                else if (c - topk_len < swa_len && c - topk_len < a.window)
-                    x = wrap_add(swa_base, c - topk_len);
-                if (c < a.width)
-                    orow[c * a.out_s1] = x;
+                else if (w < swa_len && w < a.window)
+                    x = wrap_add(swa_base, w);
+                if (c < width)
+                    ocol[k * ostep] = x;
             }
+            tcol += kAhead * tstep;
+            ocol += kAhead * ostep;
         }
         if (lane == 0)
             a.lens[t] = topk_len + swa_len;
+    }
+}
+
+// Calls f with the columns per lane of rows of `cols` columns, as a constant.
+template <typename F>
+void with_ahead(int64_t cols, F f) {
+    const int64_t n = std::max<int64_t>((cols + 63) / 64, 1), passes = (n + kMostAhead - 1) / kMostAhead;
+    switch ((n + passes - 1) / passes) {
+        case 1: return f(std::integral_constant<int, 1>());
+        case 2: return f(std::integral_constant<int, 2>());
+        case 3: return f(std::integral_constant<int, 3>());
+        case 4: return f(std::integral_constant<int, 4>());
+        case 5: return f(std::integral_constant<int, 5>());
+        case 6: return f(std::integral_constant<int, 6>());
+        case 7: return f(std::integral_constant<int, 7>());
+        default: return f(std::integral_constant<int, kMostAhead>());
     }
 }
 
@@ -195,7 +234,10 @@ extern "C" int fgv_compute_global_topk_indices_and_lens(
     a.topk = (int32_t)topk;
     a.block_size = (int32_t)block_size;
     const dim3 grid((unsigned)((num_tokens + kRowsPerBlock - 1) / kRowsPerBlock));
-    hipLaunchKernelGGL(global_topk_indices_kernel, grid, dim3(kThreads), 0, static_cast<hipStream_t>(stream), a);
+    with_ahead(topk, [&](auto n) {
+        hipLaunchKernelGGL(global_topk_indices_kernel<n.value>, grid, dim3(kThreads), 0,
+                           static_cast<hipStream_t>(stream), a);
+    });
     return launch_status();
 }
 
@@ -253,7 +295,9 @@ extern "C" int fgv_combine_topk_swa_indices(
     const int64_t workers = std::min<int64_t>(128, std::max<int64_t>(1, (per_req + kRowsPerBlock - 1) / kRowsPerBlock));
     if (num_reqs > 0x7fffffffLL / workers)
         return fail(FGV_E_TOO_LARGE, "too many requests");
-    hipLaunchKernelGGL(combine_topk_swa_kernel, dim3((unsigned)num_reqs, (unsigned)workers), dim3(kThreads), 0,
-                       static_cast<hipStream_t>(stream), a);
+    with_ahead(width, [&](auto n) {
+        hipLaunchKernelGGL(combine_topk_swa_kernel<n.value>, dim3((unsigned)num_reqs, (unsigned)workers),
+                           dim3(kThreads), 0, static_cast<hipStream_t>(stream), a);
+    });
     return launch_status();
 }

@@ -347,3 +347,28 @@ def test_gpu_rows_around_a_pass(topk):
     exp, exp_lens = oracle.combine_topk_swa_indices(loc, *args)
     got, lens = flaggems_vllm.combine_topk_swa_indices(loc.to(DEV), *(a.to(DEV) if torch.is_tensor(a) else a for a in args))
     assert torch.equal(got.cpu(), exp) and torch.equal(lens.cpu(), exp_lens)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("topk", [64, 128, 129, 193, 257, 321, 385, 449, 577, 1024])
+def test_gpu_rows_by_columns_per_lane(topk):
+    """Every count of columns per lane (one to eight, in one pass and two), for
+    both ops, from columns of a wider tensor and with every second column."""
+    import flaggems_vllm
+
+    print(f"\n[case] index rows columns topk={topk}", flush=True)
+    g = torch.Generator().manual_seed(topk)
+    T, blocks = 70, 9
+    wide = torch.randint(-1, 16 * (blocks + 1), (T, 2 * topk + 3), generator=g, dtype=I32)
+    req = torch.randint(0, 5, (T,), generator=g, dtype=I32)
+    bt = torch.randint(0, 1000, (5, blocks), generator=g, dtype=I32)
+    args = (_t([0, 30, 70]), _t([35, 3000]), _t([35, 200]), 100, 4, topk, 900, 500)
+    for cut in (slice(0, topk), slice(3, 2 * topk + 3, 2)):
+        loc, dev = wide[:, cut], wide.to(DEV)[:, cut]
+        exp, exp_lens = oracle.compute_global_topk_indices_and_lens(loc.contiguous(), req, bt, 16)
+        got, lens = flaggems_vllm.compute_global_topk_indices_and_lens(dev, req.to(DEV), bt.to(DEV), 16)
+        assert torch.equal(got.cpu(), exp) and torch.equal(lens.cpu(), exp_lens)
+        exp, exp_lens = oracle.combine_topk_swa_indices(loc.contiguous(), *args)
+        got, lens = flaggems_vllm.combine_topk_swa_indices(
+            dev, *(a.to(DEV) if torch.is_tensor(a) else a for a in args))
+        assert torch.equal(got.cpu(), exp) and torch.equal(lens.cpu(), exp_lens)
