@@ -309,19 +309,33 @@ struct PagedArgs {
     int32_t max_model_len;
     int32_t block_shift;                    // log2 of block_size where that is a power of two (SHIFT)
     int32_t vec_fill;                       // output rows 16-byte aligned, max_model_len % 4 == 0
+    int32_t rows_first;                     // grid (rows, position blocks), else (position blocks, rows)
     float fill;
 };
 
-// Paged logits: one workgroup per (row, kPagedKeys positions).
+// Paged logits: one workgroup per (row, kPagedKeys positions).  Workgroups go
+// out position block by position block (a.rows_first), so those wholly past
+// their contexts, which only fill, come last: between the others they let the
+// dispatcher stack up to three of those on one CU beside empty ones.  A block
+// starts one row further than the block before it, else a row count that is a
+// multiple of 8 keeps each row on one XCD (32 ragged rows x 65536 positions
+// 56.8 us without the turn, 50.8 with).  Row by row against this, us: 200
+// rows x 2000 23.4 -> 15.4, 600 x 1000 32.3 -> 19.8, 24 x 16384 17.3 -> 13.1,
+// 256 x 8192 57.1 -> 51.6, 32 x 65536 50.1 -> 50.5.
 constexpr int kPagedKeys = 1024;
 template <bool FP4, int HT, bool SHIFT>
 __global__ void __launch_bounds__(kThreadsM, 2)
 paged_mqa_logits_kernel(PagedArgs a) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, g = lane >> 4;
-    constexpr int kSteps = kPagedKeys / kThreadsM;
-    const int row = blockIdx.y;
-    const int n_begin = blockIdx.x * kPagedKeys;
+    uint32_t row_u = blockIdx.y, block = blockIdx.x;
+    if (a.rows_first) {
+        block = blockIdx.y;
+        row_u = blockIdx.x + block % gridDim.x;
+        row_u = row_u < gridDim.x ? row_u : row_u - gridDim.x;
+    }
+    const int row = (int)row_u;
+    const int n_begin = (int)block * kPagedKeys;
     const int n_end = min(a.max_model_len, n_begin + kPagedKeys);
     const int ctx = min(max(a.ctx[row / a.ctx_row_div], 0), a.max_model_len);
     float* out = a.out + (int64_t)row * a.o_sr;
@@ -341,78 +355,76 @@ paged_mqa_logits_kernel(PagedArgs a) {
             a.w + (int64_t)row * a.w_sr, a.w_sh, c, g);
     const int32_t* bt_row = a.bt + (int64_t)(row / a.bt_row_div) * a.bt_sr;
     const int64_t scale_off = (int64_t)a.block_size * kIdxDim;
-    // A wave takes 64 positions (four 16-key tiles) per step, kSteps steps.  The
-    // block-table entries of every step are loaded first, together; each key
-    // tile's registers then take the next step's tile as soon as the tile's own
-    // MFMAs have read them, so three tiles' loads are in flight under each
-    // tile's MFMAs and gate, with the registers of one step.  Positions from ctx
-    // on read position ctx - 1 (they are not stored).  What bounds it: the
-    // keys' HBM stream.  32 rows x 65536 positions 77.7 -> 71.8 us, 256 x 8192
-    // 81.3 -> 78.3, 4 x 2 x 3000 10.3 -> 7.8 (against all four tiles' table entries and keys loaded, then
-    // multiplied; a second step's tiles in registers of their own measured
-    // 1.6x slower than that: 184 VGPRs; the 174 here held to 168 spill: 121 us).
+    // A wave takes 64 positions (four 16-key tiles) per step.  Each key tile's
+    // registers take the next step's tile as soon as the tile's own MFMAs have
+    // read them, so three tiles' loads are in flight under each tile's MFMAs
+    // and gate, with the registers of one step; a lane holds the block and the
+    // scale of its own position, and a tile's block ids come from the lanes that
+    // hold them.  The block ids are looked up two steps ahead.  Positions from
+    // ctx on read position ctx - 1 (they are not stored).  What bounds it: the
+    // keys' HBM stream.
+    //   The steps' code is straight (the last one, which fetches nothing, is
+    // apart): with the fetches under a condition the compiler sinks every MFMA
+    // behind them, and unrolled it needs 174 VGPRs at 64 heads (117 here), two
+    // waves per SIMD for four.  Against every tile's block ids and keys loaded,
+    // then multiplied / the unrolled look-ahead, us, FP8, 64 heads: 32 rows x
+    // 65536 positions 62.7 / 58.4 / 49.0, 256 x 8192 69 / 66 / 51, 32 x 16384
+    // 20.1 / 22.7 / 17.5, 8 x 3000 10.6 / 7.5 / 7.0; 16 heads, 32 x 65536 52.3 /
+    // 45.7 / 47.3; 128 heads 78 / 73 / 63.
     const int w0 = n_begin + 64 * wave, last = ctx - 1;
     auto block_of = [&](int n) { return SHIFT ? n >> a.block_shift : (int)((uint32_t)n / (uint32_t)a.block_size); };
-    int blk[2][4];  // of this step and the next
     auto look_up = [&](int s) __attribute__((always_inline)) {
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)  // (positions past the table read its last block: the table index is clamped)
-            blk[s & 1][kt] = bt_row[min(block_of(min(w0 + 256 * s + 16 * kt + c, last)), a.max_blocks - 1)];
+        // (positions past the table read its last block: the table index is clamped)
+        return bt_row[min(block_of(min(w0 + 256 * s + lane, last)), a.max_blocks - 1)];
     };
-    look_up(0);
-    look_up(1);
+    auto row_of = [&](int block) { return a.kv + (int64_t)min(max(block, 0), a.num_blocks - 1) * a.kv_bs; };
     v8i_t b[4];
-    float ksc[4], ksc_next[4];
-    auto fetch = [&](int s, int kt) __attribute__((always_inline)) {
+    auto fetch = [&](int s, int block, int kt) __attribute__((always_inline)) {
         const int n = min(w0 + 256 * s + 16 * kt + c, last);
-        const int slot = n - block_of(n) * a.block_size;
-        const uint8_t* base = a.kv + (int64_t)min(max(blk[s & 1][kt], 0), a.num_blocks - 1) * a.kv_bs;
-        b[kt] = fp8_operand(base + (int64_t)slot * kIdxDim, g);
-        ksc_next[kt] = *reinterpret_cast<const float*>(base + scale_off + 4 * slot);
+        b[kt] = fp8_operand(
+            row_of(__shfl(block, 16 * kt + c)) + (int64_t)(n - block_of(n) * a.block_size) * kIdxDim, g);
     };
-    constexpr bool kPipe = 16 * HT < kOneQueryHeads;  // (128 heads: no registers for it)
-    if (kPipe) {
+    auto fetch_scale = [&](int s, int block) __attribute__((always_inline)) {
+        const int n = min(w0 + 256 * s + lane, last);
+        return *reinterpret_cast<const float*>(row_of(block) + scale_off + 4 * (n - block_of(n) * a.block_size));
+    };
+    const int steps = (max(min(n_end, ctx) - w0, 0) + 255) / 256;
+    int blk = look_up(0), ahead = look_up(1);  // of the step to fetch next and the one after
+    float scale = fetch_scale(0, blk);
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-            fetch(0, kt);
-    }
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) {
-        const int n0 = w0 + 256 * s;
-        if (n0 >= n_end)
-            break;
-        float v = a.fill;
-        if (n0 < ctx) {  // (wave-uniform, as is n0)
-            const bool more = kPipe && s + 1 < kSteps && n0 + 256 < ctx;
-            if (!kPipe) {
-#pragma unroll
-                for (int kt = 0; kt < 4; ++kt)
-                    fetch(s, kt);
-            }
-            if (s + 2 < kSteps)
-                look_up(s + 2);  // (over step s's entries, which its fetches have read)
-            float p[4];
-#pragma unroll
-            for (int kt = 0; kt < 4; ++kt)
-                ksc[kt] = ksc_next[kt];
-#pragma unroll
-            for (int kt = 0; kt < 4; ++kt) {
-                p[kt] = qr.gated_part(b[kt]);
-                if (more)
-                    fetch(s + 1, kt);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            // lane l: position n0 + l (its key tile g's scale sits in lane (c, g)'s ksc[g])
-            float my_ksc = ksc[0];
-#pragma unroll
-            for (int kt = 1; kt < 4; ++kt)
-                my_ksc = g == kt ? ksc[kt] : my_ksc;
-            v = reduce_scatter4(p) * my_ksc;
+    for (int kt = 0; kt < 4; ++kt)
+        fetch(0, blk, kt);
+    blk = ahead;
+    auto step = [&](int s, bool more) __attribute__((always_inline)) {
+        float p[4], next = 0.f;
+        if (more) {
+            ahead = look_up(s + 2);
+            next = fetch_scale(s + 1, blk);
         }
-        const int n = n0 + lane;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+            p[kt] = qr.gated_part(b[kt]);
+            if (more)
+                fetch(s + 1, blk, kt);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const int n = w0 + 256 * s + lane;
+        const float v = reduce_scatter4(p) * scale;
         if (n < n_end)
             out[n] = n < ctx ? v : a.fill;
-    }
+        scale = next;
+        blk = ahead;
+    };
+    // everything above has landed: else the loop would wait for the weights,
+    // the last of it, on every step, and so for the next step's keys
+    __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // vmcnt(0)
+#pragma unroll 1
+    for (int s = 0; s + 1 < steps; ++s)
+        step(s, true);
+    if (steps > 0)
+        step(steps - 1, false);
+    for (int n = w0 + 256 * steps + lane; n < n_end; n += 256)
+        out[n] = a.fill;
 }
 
 // Few queries: the four waves split each chunk's key tiles (one query per
@@ -574,7 +586,9 @@ extern "C" int fgv_fp8_fp4_paged_mqa_logits(
     a.vec_fill = aligned(logits, 16) && logits_stride_row % 4 == 0 && max_model_len % 4 == 0;
     a.fill = clean_logits ? -__builtin_inff() : 0.f;
     const bool fp4 = q_scale != nullptr;
-    const dim3 grid((uint32_t)((max_model_len + kPagedKeys - 1) / kPagedKeys), (uint32_t)rows);
+    const uint32_t blocks = (uint32_t)((max_model_len + kPagedKeys - 1) / kPagedKeys);
+    a.rows_first = blocks <= 65535;  // (a grid's second dimension holds no more)
+    const dim3 grid = a.rows_first ? dim3((uint32_t)rows, blocks) : dim3(blocks, (uint32_t)rows);
     hipStream_t st = static_cast<hipStream_t>(stream);
     switch (num_heads) {
         case 16: launch_paged<1>(fp4, shift, grid, st, a); break;

@@ -736,13 +736,13 @@ def make_paged_cache(num_blocks: int, block_size: int, gen: torch.Generator) -> 
 
 
 def make_paged_mqa_inputs(batch: int, next_n: int, avg_ctx: int, fp4: bool = False, block_size: int = 64,
-                          num_blocks: int = None, seed: int = 0):
+                          num_blocks: int = None, seed: int = 0, heads: int = MQA_HEADS):
     """(q, kv_cache, weights, context_lens [B, next_n], block_tables) as the
     reference test draws them: lengths uniform in [0.7, 1.3] x avg_ctx,
     distinct random blocks per sequence."""
     g = torch.Generator().manual_seed(seed)
-    qf = torch.randn(batch, next_n, MQA_HEADS, 128, generator=g).to(torch.bfloat16)
-    w = torch.randn(batch * next_n, MQA_HEADS, generator=g)
+    qf = torch.randn(batch, next_n, heads, 128, generator=g).to(torch.bfloat16)
+    w = torch.randn(batch * next_n, heads, generator=g)
     base = torch.randint(max(1, int(0.7 * avg_ctx)), int(1.3 * avg_ctx) + 1, (batch,), generator=g,
                          dtype=torch.int32)
     per = (base + block_size - 1) // block_size

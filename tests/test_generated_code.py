@@ -1,8 +1,7 @@
-"""Waits in the gfx950 code of the kernels whose LDS DMAs are inline assembly.
-
-The compiler counts no DMA that it did not issue itself, so where a kernel
-relies on one, or must not drain one, shows only in the assembly that hipcc
-makes of the sources (compiled here; no GPU needed)."""
+"""What shows only in the gfx950 assembly that hipcc makes of the sources
+(compiled here; no GPU needed): the waits of the kernels whose LDS DMAs are
+inline assembly, which the compiler does not count, and the registers that set
+how many waves a SIMD holds."""
 import os
 import re
 import subprocess
@@ -12,15 +11,18 @@ import pytest
 from flaggems_vllm import _native
 
 
+def _assembly(source, out):
+    flags = [f for f in _native.HIPCC_FLAGS if f not in ("-fPIC", "-shared")]
+    subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), *flags, "-S", "--cuda-device-only",
+                    f"-I{_native._INCLUDE}", f"-I{_native._CSRC}", os.path.join(_native._CSRC, source), "-o", str(out)],
+                   check=True, capture_output=True)
+    return open(out).read()
+
+
 @pytest.fixture(scope="module")
 def mla_asm(tmp_path_factory):
     """{kernel name: its instructions and labels} of sparse_mla_decode.hip."""
-    out = str(tmp_path_factory.mktemp("asm") / "mla.s")
-    flags = [f for f in _native.HIPCC_FLAGS if f not in ("-fPIC", "-shared")]
-    subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), *flags, "-S", "--cuda-device-only",
-                    f"-I{_native._INCLUDE}", f"-I{_native._CSRC}",
-                    os.path.join(_native._CSRC, "sparse_mla_decode.hip"), "-o", out], check=True, capture_output=True)
-    text, kernels = open(out).read(), {}
+    text, kernels = _assembly("sparse_mla_decode.hip", tmp_path_factory.mktemp("asm") / "mla.s"), {}
     for m in re.finditer(r"^_ZN\w*?\d+(sparse_mla_\w+?_kernel)\w*:[^\n]*\n(.*?)^\.Lfunc_end", text, re.S | re.M):
         lines = (line.split(";")[0].strip() for line in m.group(2).split("\n"))
         kernels.setdefault(m.group(1), [line for line in lines if line and not line.startswith((".p2align", ".loc"))])
@@ -64,3 +66,19 @@ def test_no_wait_drains_a_gather(mla_asm, kernel):
         assert [s[0] for s in seen] == [True, False, False]
         del seen[1]
     assert not any(waits for _, waits in seen), seen
+
+
+def test_paged_logits_registers(tmp_path):
+    """Vector registers of the paged indexer logits, which loads each key tile's
+    successor into the same registers: four waves per SIMD up to 64 heads (128
+    registers), three at 128 heads with MXFP4 queries (168), and no spills."""
+    text = _assembly("mqa_logits.hip", tmp_path / "mqa.s")
+    seen = {}
+    for m in re.finditer(r"\.name:\s+\S*paged_mqa_logits_kernelILb(\d)ELi(\d)E\S*\n(.*?)\.wavefront_size", text, re.S):
+        count, spills = (int(re.search(rf"\.vgpr_{k}:\s+(\d+)", m.group(3)).group(1)) for k in ("count", "spill_count"))
+        assert spills == 0
+        key = (m.group(1) == "1", 16 * int(m.group(2)))
+        seen[key] = max(count, seen.get(key, 0))
+    assert set(seen) == {(fp4, heads) for fp4 in (False, True) for heads in (16, 32, 64, 128)}
+    for (fp4, heads), count in seen.items():
+        assert count <= (128 if heads <= 64 else 168 if fp4 else 256), (fp4, heads, count)

@@ -441,6 +441,39 @@ def test_gpu_paged_step_edges(fp4, block_size):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("block_size", [64, 48])
+@pytest.mark.parametrize("fp4", [False, True])
+@pytest.mark.parametrize("heads", [16, 32, 128])
+def test_gpu_paged_head_counts(heads, fp4, block_size):
+    """The step edges at every head count but the 64 above, over fewer rows than
+    position blocks and with no number of rows that the turn of the blocks over
+    the rows divides."""
+    _say(f"paged mqa logits heads={heads} fp4={fp4} block_size={block_size}")
+    ctx = torch.tensor([1, 17, 64, 257, 769, 1023, 1025, 2047, 2049], dtype=torch.int32)
+    q, cache, w, _, bt = W.make_paged_mqa_inputs(9, 1, 1700, fp4=fp4, block_size=block_size, seed=23, heads=heads)
+    _check_paged(q, cache, w, ctx, bt, 2304, False, rows=torch.arange(9))
+    two = slice(4, 6)
+    q2 = (q[0][two], q[1][two] if fp4 else None)
+    _check_paged(q2, cache, w[two], ctx[two] + 4000, bt[two], 6000, True, rows=torch.arange(2))
+
+
+@pytest.mark.gpu
+def test_gpu_paged_more_blocks_than_a_grid_dimension():
+    """A max_model_len of more than 65535 position blocks."""
+    _say("paged mqa logits 65537 position blocks")
+    mml = 65536 * 1024 + 4
+    ctx = torch.tensor([70, 3000], dtype=torch.int32)
+    q, cache, w, _, bt = W.make_paged_mqa_inputs(2, 1, 2600, seed=29)
+    want, bound = oracle.paged_mqa_logits(q, cache, w, ctx, bt, 4096, True, rows=torch.arange(2))
+    got = flaggems_vllm.fp8_fp4_paged_mqa_logits((q[0].to(DEV), None), cache.to(DEV), w.to(DEV), ctx.to(DEV),
+                                                 bt.to(DEV), None, mml, clean_logits=True)
+    torch.cuda.synchronize()
+    assert got.shape == (2, mml)
+    _within(got[:, :4096].cpu(), want, bound, "65537 blocks")
+    assert bool((got[:, 4096:] == float("-inf")).all())
+
+
+@pytest.mark.gpu
 def test_gpu_pipeline_from_indexer_ops():
     """The DeepSeek-V4 indexer chain on the GPU: fused_indexer_q_rope_quant
     (FP8 and MXFP4 q, folded weights) -> indexer_k_quant_and_cache (keys into
