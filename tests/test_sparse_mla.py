@@ -1128,3 +1128,27 @@ def test_pieces_rule():
         for extra in (0, 192, 512, 1024, 1888):
             for heads in (64, 128):
                 assert f(batch, 1, heads, 128, extra, 1 << 20) <= 64 << 20 or grid(batch, 1, heads, 128, extra) == 1
+
+
+@pytest.mark.gpu
+def test_gpu_split_grid_more_items_than_a_grid_of_merges():
+    """Long lists over 1,056,000 items: 16 merging workgroups each would be
+    more threads than a grid holds.  Every row has the same query and entry (so
+    the outputs, which all go to one place, are the same), but one in nine
+    attends nothing, which the combine kernel writes."""
+    import flaggems_vllm
+
+    print("\n[case] sparse MLA split grid, 1056000 items", flush=True)
+    B, SQ = 8000, 132
+    w = W.make_mla_workload(batch=1, topk=2048, num_pages=4, seed=99, q_scale=0.1)
+    d = w.to(DEV)
+    lens = torch.ones(B, dtype=torch.int32, device=DEV)
+    lens[8::9] = 0
+    out = torch.empty(1, 1, 64, 512, dtype=torch.bfloat16, device=DEV)
+    _, lse = flaggems_vllm.flash_mla_with_kvcache(
+        d.q.expand(B, SQ, 64, 512), d.k_cache, None, None, 512, _meta(), is_fp8_kvcache=True,
+        indices=d.indices.expand(B, SQ, 2048), topk_length=lens, out=out.expand(B, SQ, 64, 512))
+    torch.cuda.synchronize()
+    some = lse[0, :, 0]
+    assert bool(torch.isfinite(some).all())
+    assert bool((lse[lens == 1] == some[None, :, None]).all()) and bool((lse[lens == 0] == float("inf")).all())
