@@ -2048,7 +2048,11 @@ int mla_decode(FGV_MLA_PARAMS, void* workspace, int64_t workspace_bytes, void* s
         split_bytes(batch, seq_q, num_heads, topk, extra_k_cache ? extra_topk : 0, need_expand > 0);
     const int64_t have = workspace ? workspace_bytes : 0;
     const bool use_expand = need_expand > 0 && have >= need_expand + need_split;
-    const bool use_split = need_split > 0 && have >= need_split + (use_expand ? need_expand : 0);
+    const bool pieces = mla_grid(batch, seq_q, num_heads, topk, extra_k_cache ? extra_topk : 0) == kGridPieces;
+    // (calls that may be cut into pieces take any workspace, as they did when
+    // they had no use for one; a misaligned one holds no pieces)
+    const bool use_split = need_split > 0 && have >= need_split + (use_expand ? need_expand : 0) &&
+                           !(pieces && !aligned(workspace, 256));
     if ((use_expand || use_split) && !aligned(workspace, 256))
         return fail(FGV_E_MISALIGNED, "workspace must be 256-byte aligned");
     uint8_t* ws = static_cast<uint8_t*>(workspace);
@@ -2067,7 +2071,7 @@ int mla_decode(FGV_MLA_PARAMS, void* workspace, int64_t workspace_bytes, void* s
             return rc;
         ws += need_expand;
     }
-    if (use_split && mla_grid(batch, seq_q, num_heads, topk, extra_k_cache ? extra_topk : 0) == kGridPieces) {
+    if (use_split && pieces) {
         a.pieces = (int32_t)pieces_of(items, topk, extra_k_cache ? extra_topk : 0);
         const int64_t widest = chunks_of(topk) + chunks_of(extra_k_cache ? extra_topk : 0);
         a.piece_chunks = (int32_t)((widest + a.pieces - 1) / a.pieces);

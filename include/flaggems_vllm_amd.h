@@ -397,7 +397,9 @@ int fgv_sparse_mla_decode_model1(
  * extra_num_entries is extra_num_blocks * extra_page_size (0 without an extra
  * cache).  0 means the workspace argument is ignored.  Passing no workspace
  * (NULL or too small) always works: a workspace too small for both parts drops
- * the expansion first, then the split (one workgroup per item).
+ * the expansion first, then the split or the pieces (one workgroup per item).
+ * A workspace that is not 256-byte aligned holds no pieces, and is refused
+ * (FGV_E_MISALIGNED) for the other two.
  */
 int64_t fgv_sparse_mla_decode_workspace_bytes(int64_t batch, int64_t seq_q, int64_t num_heads,
                                               int64_t topk, int64_t extra_topk, int64_t extra_num_entries);

@@ -1152,3 +1152,33 @@ def test_gpu_split_grid_more_items_than_a_grid_of_merges():
     some = lse[0, :, 0]
     assert bool(torch.isfinite(some).all())
     assert bool((lse[lens == 1] == some[None, :, None]).all()) and bool((lse[lens == 0] == float("inf")).all())
+
+
+@pytest.mark.gpu
+def test_gpu_pieces_misaligned_workspace():
+    """A call that cuts its items only where it may leaves them whole when the
+    workspace is not 256-byte aligned, as it does without one."""
+    from flaggems_vllm import _native
+
+    print("\n[case] sparse MLA pieces, misaligned workspace", flush=True)
+    w = _pieces_case("least")
+    d = w.to(DEV)
+    L = _native.lib()
+    entries = d.extra_k_cache.shape[0] * d.extra_k_cache.shape[1]
+    nbytes = L.fgv_sparse_mla_decode_workspace_bytes(1, 1, 64, 256, 64, entries)
+    assert _grid(w) == 3 and nbytes > 0
+    ws = torch.empty(nbytes + 256, dtype=torch.uint8, device=DEV)
+    out = torch.full((1, 1, 64, 512), float("nan"), dtype=torch.bfloat16, device=DEV)
+    lse = torch.full((1, 64, 1), float("nan"), device=DEV)
+    ptr = lambda t: t.data_ptr() if t is not None else None
+    rc = L.fgv_sparse_mla_decode_model1(
+        d.q.data_ptr(), *d.q.stride()[:3], d.k_cache.data_ptr(), d.k_cache.stride(0), *d.k_cache.shape[:2],
+        d.indices.data_ptr(), *d.indices.stride()[:2], 256, None, d.extra_k_cache.data_ptr(),
+        d.extra_k_cache.stride(0), *d.extra_k_cache.shape[:2], d.extra_indices.data_ptr(),
+        *d.extra_indices.stride()[:2], 64, None, ptr(d.attn_sink), 512 ** -0.5, out.data_ptr(), *out.stride()[:3],
+        lse.data_ptr(), *lse.stride()[:2], 1, 1, 64, ws.data_ptr() + 16, nbytes,
+        torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert rc == 0, L.fgv_last_error()
+    uncut, uncut_lse, _ = _gpu_raw(w, workspace=False)
+    assert torch.equal(out.cpu().view(torch.int16), uncut.view(torch.int16)) and torch.equal(lse.cpu(), uncut_lse)
