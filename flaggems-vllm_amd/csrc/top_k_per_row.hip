@@ -555,10 +555,14 @@ top_k_per_row_kernel(TopkArgs a) {
 // per value; LDS holds the histogram only.  Kept values are counted and placed
 // by one scan over the threads, so a row's output order is fixed.  What bounds
 // it: the scans' barriers and the histogram atomics (randn rows crowd into few
-// bins).  Measured against the row in LDS (graph
-// replays, randn rows, k 512, us): 24 x 16384 17.1 -> 14.1, 1024 x 9000 28.1 ->
-// 25.8, 2048 x 16384 79.8 -> 63.5, 64 x 4096 10.2 -> 8.6, 16383 x 4095 143 ->
-// 113, 512 x 9000 15.4 -> 15.9.
+// bins).  Every level walks all slots, so what a slot costs there counts: an
+// empty-slot test on each level and one output pass for ties and no ties held
+// a 64-bit mask per slot (71 spilled scalars at 32 slots), and 512 rows, two
+// per CU, ran slower than in LDS.  Measured with the row in LDS / with those
+// masks / as here (graph replays, randn rows, k 512, us): 24 x 16384 17.1 /
+// 15.1 / 10.8, 64 x 4096 10.3 / 8.5 / 7.2, 512 x 9000 15.4 / 15.9 / 12.7, 512 x
+// 16384 22.7 / 22.7 / 17.0, 1024 x 9000 27.8 / 25.7 / 21.8, 4096 x 4096 39.8 /
+// 32.3 / 28.3, 24 x 9000 of every third column 12.3 / 11.8 / 9.3.
 template <int THREADS, int N>
 __device__ __forceinline__ void row_select(const TopkArgs& a, int32_t r, int32_t start, int32_t len, uint32_t* hist,
                                            uint32_t* wsum, int32_t* sel) {
@@ -626,11 +630,11 @@ __device__ __forceinline__ void row_select(const TopkArgs& a, int32_t r, int32_t
         return b;
     };
     const uint32_t b1 = level([&](int n) { return key[n] != 0; }, [&](int n) { return key[n] >> 21; });
-    const uint32_t b2 = level([&](int n) { return key[n] != 0 && key[n] >> 21 == b1; },
-                              [&](int n) { return (key[n] >> 10) & 0x7ff; });
+    // (a value's key is at least -inf's, 0x007fffff, so b1 > 0 and no empty slot
+    // is counted further on)
+    const uint32_t b2 = level([&](int n) { return key[n] >> 21 == b1; }, [&](int n) { return (key[n] >> 10) & 0x7ff; });
     const uint32_t p2 = b1 << 11 | b2;
-    const uint32_t b3 = level([&](int n) { return key[n] != 0 && key[n] >> 10 == p2; },
-                              [&](int n) { return key[n] & 0x3ff; });
+    const uint32_t b3 = level([&](int n) { return key[n] >> 10 == p2; }, [&](int n) { return key[n] & 0x3ff; });
     const uint32_t key_t = p2 << 10 | b3;
     // the values equal to the k-th largest: all of them, or the `need` with the
     // smallest indices, found as the largest of 8 kBins - 1 - index
@@ -644,24 +648,29 @@ __device__ __forceinline__ void row_select(const TopkArgs& a, int32_t r, int32_t
                                   [&](int n) { return rev(n) & 7; });
         last = 8 * kBins - 1 - (int32_t)(c1 << 3 | c2);
     }
-    auto kept = [&](int n) { return key[n] > key_t || (key[n] == key_t && index(n) <= last); };
-    uint32_t mine = 0, total;
+    auto place = [&](auto&& kept) __attribute__((always_inline)) {
+        uint32_t mine = 0, total;
 #pragma unroll
-    for (int n = 0; n < N + 2; ++n)
-        mine += kept(n) ? 1u : 0u;
-    uint32_t p = B::scan(mine, wsum, total);
+        for (int n = 0; n < N + 2; ++n)
+            mine += kept(n) ? 1u : 0u;
+        int32_t* o = orow + (int64_t)B::scan(mine, wsum, total) * a.os1;
 #pragma unroll
-    for (int n = 0; n < N + 2; ++n)
-        if (kept(n)) {
-            orow[(int64_t)p * a.os1] = index(n);
-            ++p;
-        }
+        for (int n = 0; n < N + 2; ++n)
+            if (kept(n)) {
+                *o = index(n);
+                o += a.os1;
+            }
+    };
+    if (last == 0x7fffffff)
+        place([&](int n) { return key[n] >= key_t; });
+    else
+        place([&](int n) { return key[n] > key_t || (key[n] == key_t && index(n) <= last); });
 }
 
 // Each row takes the fewest slots, in steps of 4, that hold it: every pass walks
 // all of them.  (With the launch's most for every row, ragged prefill rows of
-// 2400 to 4096 values in 9800 columns ran slower than in LDS; in steps of 8,
-// 512 rows of 9000 17.1 us, 15.4 in LDS.)
+// 2400 to 4096 values in 9800 columns ran slower than in LDS; in steps of 8
+// 512 rows of 9000 took 17.1 us where steps of 4 took 15.9.)
 template <int THREADS, int N, int MAXN>
 __device__ __forceinline__ void fewest_slots(const TopkArgs& a, int32_t r, int32_t start, int32_t len, uint32_t* hist,
                                              uint32_t* wsum, int32_t* sel) {

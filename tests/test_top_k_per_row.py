@@ -377,3 +377,35 @@ def test_gpu_row_slots(width):
     starts = torch.tensor([min(i % 5, width - n) for i, n in enumerate(lens)], dtype=I32)
     ends = starts + torch.tensor(lens, dtype=I32)
     _run_prefill(x, starts, ends, k, range(len(lens)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("stride", [1, 3])
+@pytest.mark.parametrize("width", [4000, 8000, 16000])
+def test_gpu_row_slots_low_values_and_strides(width, stride):
+    """Rows in registers, every third column of a wider tensor among them, either
+    side of a slot count: ties at the k-th that go by index, -inf at the k-th
+    (the lowest key, which the empty slots' must stay below), rows of -inf
+    alone, and NaN."""
+    print(f"\n[case] top-k row slots width={width} stride={stride}", flush=True)
+    threads, k = (256 if width == 4000 else 512), 300
+    lens = [width, width - 1] + [s * threads + d for s in (4, 8, width // threads) for d in (-1, 0, 1)]
+    lens = [n for n in lens for _ in range(4)]
+    g = torch.Generator().manual_seed(width + stride)
+    x = torch.randn(len(lens), width, generator=g)
+    x[1::4] = torch.randint(0, 3, x[1::4].shape, generator=g).float()
+    x[2::4, 100:] = float("-inf")                  # fewer than k finite values
+    x[3::4] = float("-inf")
+    x[3::8, ::50] = float("nan")
+    wide = torch.zeros(len(lens), width * stride)
+    wide[:, ::stride] = x
+    ends = torch.tensor([min(n, width) for n in lens], dtype=I32)
+    idx = torch.full((len(lens), k), -7, dtype=I32, device=DEV)
+    import flaggems_vllm
+
+    dl = wide.to(DEV)[:, ::stride]
+    flaggems_vllm.top_k_per_row_prefill(dl, torch.zeros_like(ends).to(DEV), ends.to(DEV), idx, len(lens), dl.stride(0),
+                                        dl.stride(1), k)
+    torch.cuda.synchronize()
+    rows = list(range(len(lens)))
+    _check_rows(idx, x, k, rows, oracle.top_k_per_row(x, k, row_starts=torch.zeros_like(ends), row_ends=ends, rows=rows))
