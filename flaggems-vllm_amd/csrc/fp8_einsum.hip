@@ -270,7 +270,11 @@ __global__ void __launch_bounds__(64 * KS) fp8_einsum_skinny_kernel(EinsumArgs a
 // graph replays with the inverse-RoPE quantisation before it, us, h 8, r 4096:
 // b 700 91.2 -> 73.9, b 8192 465 -> 460; h 16, r 7168: b 200, split, 82.5 ->
 // 69.5, b 2500 514 -> 506.  B's and the scales' operands in a second register
-// set spill the 256-row kernel: 1457 us at b 8192.)
+// set spill the 256-row kernel: 1457 us at b 8192.)  The last block reads
+// nothing ahead and has code of its own: with its reads in the loop, unused,
+// short sums lost more than reading ahead gave (h 8, b 2500, the product alone,
+// us: r 128 19.7 before, 20.8 with them, 20.0 here; r 256 25.2 / 26.1 / 25.2; r
+// 4096 143 / 131.2 / 130.6).
 constexpr int kStages4 = 3;  // LDS stages of the 256-row tiles (49 KB each)
 constexpr int kStages2 = 3;  // LDS stages of the 128-row tiles (33 KB each)
 
@@ -409,8 +413,8 @@ __global__ void __launch_bounds__(128 * MW) fp8_einsum_tile_kernel(EinsumArgs a,
     // kb + 3 - into block kb's stage - and the LDS reads of block kb + 1's
     // operands between them, each operand after its last use.  A product is
     // scaled into the accumulator two MFMAs later.
-    auto step = [&](int kb, int at) __attribute__((always_inline)) {
-        const bool next = kb + 1 < kb_hi, send = kb + NS < kb_hi;
+    auto step = [&](int kb, int at, bool next) __attribute__((always_inline)) {
+        const bool send = next && kb + NS < kb_hi;
         const uint8_t* nxt = st[at + 1 < NS ? at + 1 : 0];
         const uint32_t dst = lds_addr(st[at]);
         if (next) {
@@ -432,15 +436,16 @@ __global__ void __launch_bounds__(128 * MW) fp8_einsum_tile_kernel(EinsumArgs a,
                 sx[i & 1] = v4f_t{X[i].x * y, X[i].y * y, X[i].z * y, X[i].w * y};
             if (send && u % kEvery == kEvery - 1 && u / kEvery <= kPer)
                 issue(kb + NS, dst, u / kEvery);
-            // (after the last block these read a stage's old bytes, unused)
-            if (j == 3) {
-                read_a(nxt, i);
-                read_x(nxt, i);
+            if (next) {
+                if (j == 3) {
+                    read_a(nxt, i);
+                    read_x(nxt, i);
+                }
+                if (i == 3)
+                    read_b(nxt, j);
+                if (u == 2)
+                    read_y(nxt);
             }
-            if (i == 3)
-                read_b(nxt, j);
-            if (u == 2)
-                read_y(nxt);
             if (u >= 2)
                 scale_in(u - 2);
             __builtin_amdgcn_sched_barrier(0);
@@ -477,10 +482,12 @@ __global__ void __launch_bounds__(128 * MW) fp8_einsum_tile_kernel(EinsumArgs a,
         read_y(st[0]);
     }
     int at = 0;
-    for (int kb = kb_lo; kb < kb_hi; ++kb) {
-        step(kb, at);
+    for (int kb = kb_lo; kb + 1 < kb_hi; ++kb) {
+        step(kb, at, true);
         at = at + 1 < NS ? at + 1 : 0;
     }
+    if (kb_lo < kb_hi)
+        step(kb_hi - 1, at, false);
 
     if (gridDim.z > 1) {
         float* ps = part + (int64_t)blockIdx.z * a.b * a.h * a.d;

@@ -330,6 +330,18 @@ def test_gpu_tiled_edges(b):
     _check(res, x, xs, y, ys, torch.bfloat16)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("blocks", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("b,h", [(200, 3), (2100, 8)])
+def test_gpu_tiled_few_blocks(b, h, blocks):
+    """Fewer K blocks than LDS stages, as many and more, on both tile shapes
+    (128 rows for b = 200, 256 for 2100 x 8 heads)."""
+    print(f"\n[case] fp8_einsum tiled b={b} blocks={blocks}", flush=True)
+    x, xs, y, ys = random_inputs(b, h, 128 * blocks, 512, seed=10 * b + blocks)
+    res = _run(x.to(DEV), xs.to(DEV), y.to(DEV), ys.to(DEV))
+    _check(res, x, xs, y, ys, torch.bfloat16, rows=torch.cat([torch.arange(0, b, 37), torch.tensor([b - 1])]))
+
+
 def _layout(kind, x, xs, y, ys):
     b, h, r = x.shape
     if kind == "vllm":  # head-major x, scales with strides (1, 8, 4)-like
