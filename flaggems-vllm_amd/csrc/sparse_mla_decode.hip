@@ -87,7 +87,6 @@ constexpr int kMaxSplitRows = 8000;
 // balance outweighs the partials it writes.
 constexpr int kSplitMinChunks = 64;
 constexpr int kPieceMinChunks = 2;                            // pieces mode: chunks per piece, at least
-constexpr int kPieceMost = 18;                                // and pieces per item, at most
 constexpr float kRescaleSlack = 8.0f;                         // log2 of the largest probability
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -128,8 +127,8 @@ struct MlaArgs {
     int32_t pair_cus;
     int32_t order_windows;
     // pieces mode: the most pieces per item, each with a slot of `partials`,
-    // the most chunks of a piece, and 2^16 over that, rounded up past it
-    int32_t pieces, piece_chunks, piece_mul;
+    // and the most chunks of an item that stays whole
+    int32_t pieces, whole_chunks;
 };
 
 // K tile addressing: 16-byte block b of row r at r * kKRowBytes + 16 b, rows
@@ -1237,27 +1236,26 @@ sparse_mla_decode_split_kernel(MlaArgs a) {
 //
 // An item is a serial chain of chunks (about 2 us each), so a decode batch of
 // a few rows ran one long chain per row on a few CUs while the others idled.
-// Here an item is cut into the fewest contiguous runs of at most
-// a.piece_chunks chunks, one workgroup each (at most a.pieces; shorter runs
-// would shorten nothing, the longest item's set the time), but one chunk more
-// is not worth two slots.  An item of one piece is finished by its workgroup, the others leave fp32
-// partial slots (item, piece) that sparse_mla_merge_kernel combines in piece
-// order.  The cut depends on the item's own lengths and, through
-// a.piece_chunks, on how many items the call has and how wide its lists are:
-// a row gives other low bits in a batch of another size.  What bounds it now:
-// the first chunk's chain of dependent loads (length, index, cache row) and
-// 128 KiB written and read back per slot.
+// Here an item of more than a.whole_chunks chunks is cut into up to a.pieces
+// contiguous runs of at least kPieceMinChunks, one workgroup each.  An item of
+// one piece is finished by its workgroup, the others leave fp32 partial slots
+// (item, piece) that sparse_mla_merge_kernel combines in piece order.  The cut
+// depends on the item's own lengths and, through a.pieces and a.whole_chunks,
+// on how many items the call has and how wide its lists are: a row gives other
+// low bits in a batch of another size.  What bounds it now: the first chunk's
+// chain of dependent loads (length, index, cache row) and 128 KiB written and
+// read back per slot.
 //   Measured against whole items (graph replays over 3 input sets, us per call,
 // top-k 128 + 512): all lengths full, 1 / 24 / 64 / 100 / 128 rows
-// 45.8 / 47.5 / 48.0 / 48.5 / 48.9 -> 14.7 / 26.3 / 31.6 / 40.3 / 43.0; ragged, 24 /
-// 64 / 100 rows 44.2 / 47.3 / 47.5 -> 23.1 / 27.7 / 37.0; 128 + 1856 at 24 rows 134
-// -> 33.4.  What it costs where no row is cut is the merge's launch: every row
-// of 5 chunks, 24 / 100 rows 15.5 / 17.3 -> 17.0 / 19.2 (27.3 at 100 rows with
-// every row of 4 chunks or more cut), of one chunk 7.2 / 8.0 -> 9.1 / 10.5.
+// 45.9 / 47.5 / 48.1 / 48.5 / 48.9 -> 14.6 / 28.7 / 31.4 / 40.3 / 43.1; ragged, 24 /
+// 64 / 100 rows 44.2 / 47.4 / 47.6 -> 23.6 / 28.9 / 36.5; 128 + 1856 at 24 rows 134
+// -> 33.3.  What it costs rows that are short beside the call's widths: the
+// merge's launch where none is cut (every row of one chunk, 24 / 100 rows 7.2 /
+// 8.0 -> 9.1 / 10.4, of 5 chunks, 100 rows 17.3 -> 19.2 and, with every row of 4
+// chunks or more cut, 27.3), the slots where they are (24 rows of 5 chunks 15.5
+// -> 18.6).
 __device__ __forceinline__ int item_pieces(const MlaArgs& a, int chunks) {
-    const int n = __builtin_amdgcn_readfirstlane(chunks), most = a.piece_chunks;
-    // ceil(n / most); exact for n < 64 (a division took 0.2 us of the chain)
-    return n <= most + 1 ? 1 : ((n + most - 1) * a.piece_mul) >> 16;
+    return chunks <= a.whole_chunks ? 1 : max(1, min(a.pieces, chunks / kPieceMinChunks));
 }
 
 __global__ void __launch_bounds__(kThreads, 2)
@@ -1850,48 +1848,40 @@ bool pair_fits(int64_t batch, int64_t items, int64_t topk, int64_t extra_topk) {
 }
 
 // Pieces per item (1: no cut).  Lists shorter than the split grid's but of
-// more than kPieceMinTotal chunks are cut while about one workgroup per CU has
-// work (two, for lists of kPieceLongChunks over more than a quarter as many
-// items as CUs).
-//
-// Into how many: piece_cost for lists of the call's widths at their fullest,
-// the cheapest.  In units of 0.07 us, 28 per chunk of a piece (33 with two
-// workgroups on a CU), 3 per piece of an item, and per slot of the call half
-// of what it takes when every list is full, 0.5 (0.9 past one per CU): ragged
-// batches leave about half of them empty, and cutting a little more than full
-// lists want costs those less than cutting too little costs ragged ones.
-// Whether at all: the chunks that leave the chain (2.1 us each; a unit of
-// 0.06 us here) against 4 us for the merge and 0.06 us per slot, half as much
-// again past one slot per CU.
-//   Measured with all lists full, us in 1 / 2 / 3 / 4 / 5 / 10 pieces: 24 items
-// of 20 chunks 44.0 / 32.2 / 28.1 / 26.1 / 26.1 / 28.5 (5 taken), 48 items of 10
-// chunks 25.0 / 26.2 / 26.3 / 26.5 / 28.1 / - (whole), 100 items of 36 chunks
-// 76.4 / 54.7 / 54.1 / 49.8 / - / - (4 taken), 248 items of 36 chunks 79.7 /
-// 84.0 (whole), of 62 chunks 128.0 / 118.1 (2 taken).
+// more than kPieceMinTotal chunks, over at most half as many items as CUs (at
+// most as many, for lists of kPieceLongChunks), are cut so that about one
+// workgroup per CU (two, for the latter) has work, if the chunks that leave
+// the chain are worth the slots: a chunk off the chain saves about 2.1 us, the
+// merge costs about 4 us and 0.06 us per slot, half as much again past one
+// slot per CU (measured from 2 to 496 slots).  128 + 192 entries at 2 / 24 /
+// 100 rows: 25.3 -> 13.8, 26.2 -> 23.6, and 27.6 against 30.7 us cut, which the
+// rule leaves whole; 128 + 512 at 130 / 200 rows 48.7 / 49.3 against 45.9 / 55.3
+// us in two pieces, left whole; 128 + 1024 at 100 rows 81.4 us whole, 57.5
+// with one workgroup per CU and 51.3 with two, while 24 rows take 30.2 with
+// one and 34.7 with two, at 200 rows 77.3 whole and 78.0 cut, at 248 rows 79.7
+// and 84.0, left whole.
 constexpr int64_t kPieceMinTotal = 8;
 constexpr int64_t kPieceLongChunks = 32;
 constexpr int64_t kPieceMaxSlots = 496;  // with their headers below the no-allocation entry point's 64 MiB
-
-int piece_cost(int items, int chunks, int pieces, int cus) {
-    const int slots = items * pieces, over = max(slots - cus, 0);
-    return (over ? 33 : 28) * ((chunks + pieces - 1) / pieces) + 3 * pieces + (5 * slots + 4 * over) / 10;
-}
 
 int64_t pieces_of(int64_t items, int64_t topk, int64_t extra_topk) {
     const int64_t chunks = chunks_of(topk) + chunks_of(extra_topk), cus = cu_count();
     if (chunks <= kPieceMinTotal || chunks >= kSplitMinChunks || items > cus)
         return 1;
     const bool two = 4 * items > cus && chunks >= kPieceLongChunks;
-    const int64_t most = min(min(min(two ? 2 * cus : cus, kPieceMaxSlots) / items, chunks / kPieceMinChunks),
-                             (int64_t)kPieceMost);
-    if (most < 2)
-        return 1;
-    int n = 2;
-    for (int s = 3; s <= most; ++s)
-        if (piece_cost((int)items, (int)chunks, s, (int)cus) < piece_cost((int)items, (int)chunks, n, (int)cus))
-            n = s;
+    const int64_t n = min(min(two ? 2 * cus : cus, kPieceMaxSlots) / items, chunks / kPieceMinChunks);
     const int64_t slots = n * items, over = max(slots - cus, (int64_t)0);
-    return 35 * chunks * (n - 1) > n * (67 + slots + over / 2) ? n : 1;
+    return n > 1 && 35 * chunks * (n - 1) > n * (67 + slots + over / 2) ? n : 1;
+}
+
+// The most chunks of an item that stays whole in a call cut into `pieces`: as
+// many as a piece of its longest possible item has, so that it does not set
+// the time beside that one, and from 48 items on, whose slots cost more than a
+// chunk of the chain, one more.  Longer rows are cut however many of them there
+// are: 64 rows of 8 chunks take 23.1 us whole and 28.2 cut, but 64 ragged ones
+// of 128 + 512 32.8 with rows of up to 9 chunks whole and 28.9 as here.
+int64_t whole_chunks(int64_t items, int64_t pieces, int64_t chunks) {
+    return (chunks + pieces - 1) / pieces + (items >= 48 ? 1 : 0);
 }
 
 // The grid a call runs when it gets the workspace it asks for (a call whose
@@ -2035,8 +2025,7 @@ int mla_decode(FGV_MLA_PARAMS, void* workspace, int64_t workspace_bytes, void* s
     a.pair_cus = 0;
     a.order_windows = 0;
     a.pieces = 0;
-    a.piece_chunks = 0;
-    a.piece_mul = 0;
+    a.whole_chunks = 0;
     const int64_t items = batch * seq_q * a.head_blocks;
     hipStream_t st = static_cast<hipStream_t>(stream);
     // Workspace: [expanded extra cache][partial slots][row prefix sums].  A
@@ -2074,8 +2063,7 @@ int mla_decode(FGV_MLA_PARAMS, void* workspace, int64_t workspace_bytes, void* s
     if (use_split && pieces) {
         a.pieces = (int32_t)pieces_of(items, topk, extra_k_cache ? extra_topk : 0);
         const int64_t widest = chunks_of(topk) + chunks_of(extra_k_cache ? extra_topk : 0);
-        a.piece_chunks = (int32_t)((widest + a.pieces - 1) / a.pieces);
-        a.piece_mul = 65536 / a.piece_chunks + 1;
+        a.whole_chunks = (int32_t)whole_chunks(items, a.pieces, widest);
         a.partials = reinterpret_cast<float*>(ws);
         hipLaunchKernelGGL(sparse_mla_decode_pieces_kernel, dim3((unsigned)(items * a.pieces)), dim3(kThreads), 0, st,
                            a);
