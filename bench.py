@@ -28,6 +28,15 @@ METRIC = "tokens/s and achieved HBM GB/s (% of roofline) at T=8192, H=64, D=512"
 HBM_PEAK_GBPS = 8000.0
 PROFILES = os.path.join(ROOT, "profiles")
 
+# fgv_sparse_mla_decode_grid's values: the kernel, and what the config line says of its schedule
+MLA_GRIDS = {
+    0: ("sparse_mla_decode_kernel", "one workgroup per (row, 64-head block): {items} items on {cus} CUs, {order}"),
+    1: ("sparse_mla_decode_split_kernel", "balanced split grid + combine kernel"),
+    2: ("sparse_mla_decode_pair_kernel", "paired grid: one 8-wave workgroup per CU, both halves on each item, "
+                                         "a short item after a long one"),
+    3: ("sparse_mla_decode_pieces_kernel", "items cut into pieces, a workgroup each, + merge kernel"),
+}
+
 
 def parse_args():
     ap = argparse.ArgumentParser()
@@ -734,8 +743,7 @@ def main():
         expanded = entries > 0 and need == entries * 1024 + (0 if grid == 3 else slots)
         if grid == 3 and expanded:
             grid = 0
-        kernel = {0: "sparse_mla_decode_kernel", 1: "sparse_mla_decode_split_kernel",
-                  2: "sparse_mla_decode_pair_kernel", 3: "sparse_mla_decode_pieces_kernel"}[grid]
+        kernel, schedule = MLA_GRIDS[grid]
         workload = (f"mla_{args.mla_case}" + (f"_b{B}" if args.mla_batch else "")
                     + (f"_h{HQ}" if args.mla_heads else ""))
         case = W.MLA_CASES[args.mla_case]
@@ -751,10 +759,7 @@ def main():
                                  f"of {case['extra_page']}" if "extra_topk" in case else ""),
                   "batch": B, "seq_q": SQ, "num_heads": HQ, "attended_entries": w_cpu.used_tokens(),
                   "flops_per_call": flops_call,
-                  "schedule": {0: f"one workgroup per (row, 64-head block): {items} items on {cus} CUs, {order}",
-                               1: "balanced split grid + combine kernel",
-                               2: "paired grid: one 8-wave workgroup per CU, both halves on each item, "
-                                  "a short item after a long one"}[grid]
+                  "schedule": schedule.format(items=items, cus=cus, order=order)
                               + ("; extra cache expanded to bf16 once per call" if expanded else "")}
     elif args.op == "indexer_k":
         # indexer key quantise + insert at the reference benchmark's shapes

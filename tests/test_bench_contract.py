@@ -32,3 +32,13 @@ def test_rotating_cycles_through_every_set():
     for _ in range(13):
         step()
     assert calls == [i % 6 for i in range(13)]
+
+
+def test_every_mla_grid_has_a_kernel_and_a_schedule():
+    from flaggems_vllm import _native
+
+    grid = _native.lib().fgv_sparse_mla_decode_grid
+    seen = {grid(b, 1, 64, 128, extra) for b in (1, 24, 200, 300, 512, 2000) for extra in (0, 512, 8192)}
+    assert seen == {0, 1, 2, 3} == set(bench.MLA_GRIDS)
+    for kernel, schedule in bench.MLA_GRIDS.values():
+        assert kernel.startswith("sparse_mla_decode") and schedule.format(items=1, cus=256, order="in order")
