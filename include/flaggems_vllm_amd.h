@@ -393,7 +393,14 @@ int fgv_sparse_mla_decode_model1(
  *     items (at most one per CU, or half as many) whose extra cache is not
  *     expanded are cut into up to one or two pieces per CU, and a merge kernel
  *     combines them.  At most 496 slots, which also fit the 64 MiB scratch of
- *     the no-allocation entry point.
+ *     the no-allocation entry point.  Rows that are short beside topk +
+ *     extra_topk stay whole.
+ * A row cut by the split or into pieces is summed part by part, and where it is
+ * cut follows from the whole call: the split's cuts from every row's length, the
+ * pieces' from the number of items and the widths topk and extra_topk.  So such
+ * a row's low bits differ between batches; the same call gives the same bits.
+ * Without a workspace, and below 2048 entries (from there on the paired grid sums
+ * a row in two halves), they depend on the row alone.
  * extra_num_entries is extra_num_blocks * extra_page_size (0 without an extra
  * cache).  0 means the workspace argument is ignored.  Passing no workspace
  * (NULL or too small) always works: a workspace too small for both parts drops
